@@ -19,18 +19,6 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
-// x * (1 + erf(x / sqrt 2)) / 2 (model.rs:312-314) with the device library's
-// erff (correctly rounded to within 2 ulp).
-__device__ __forceinline__ float gelu_erf(float x) {
-  return x * (1.0f + erff(x / 1.41421356237309515f)) / 2.0f;
-}
-
-__device__ __forceinline__ float activate(float x, int act) {
-  if (act == kActRelu) return fmaxf(x, 0.0f);
-  if (act == kActGelu) return gelu_erf(x);
-  return x;
-}
-
 // One wavefront per output column c: source column map ? map[c] : c of x
 // (leading dimension ldx), LayerNorm over its d features (layer_norm_host,
 // model.rs:387-422: mean, then the mean of squared deviations, then

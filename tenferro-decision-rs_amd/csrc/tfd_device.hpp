@@ -173,6 +173,18 @@ __device__ __forceinline__ void buffer_store4_nt(f32x4 v, __amdgpu_buffer_rsrc_t
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned int, v), r, voff, soff, kCacheNT);
 }
 
+// x * (1 + erf(x / sqrt 2)) / 2 (laya-infer model.rs:312-314) with the device
+// library's erff (correctly rounded to within 2 ulp).
+__device__ __forceinline__ float gelu_erf(float x) {
+  return x * (1.0f + erff(x / 1.41421356237309515f)) / 2.0f;
+}
+
+__device__ __forceinline__ float activate(float x, int act) {
+  if (act == 1) return fmaxf(x, 0.0f);  // kActRelu
+  if (act == 2) return gelu_erf(x);     // kActGelu
+  return x;
+}
+
 __device__ __forceinline__ float wave_max_f(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));

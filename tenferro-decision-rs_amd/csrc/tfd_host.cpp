@@ -17,6 +17,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -61,6 +62,7 @@ struct tfd_ctx {
   DevBuf kp;          // Jeff normalized + rotated keys
   DevBuf layer;       // intermediates of the layer entries (projections, attention output)
   DevBuf model;       // activations and token inputs of the model forward
+  DevBuf planes;      // fp16 planes of the linears' operands
   std::vector<uint8_t> model_host;  // packed token inputs of the last model forward
   bool model_inflight = false;      // an asynchronous forward may still read model_host
   rocblas_handle blas = nullptr;  // the layer entries' GEMMs, on `stream`
@@ -651,6 +653,105 @@ int gemm(tfd_ctx *c, bool ta, bool tb, size_t m, size_t n, size_t k, const float
   return TFD_OK;
 }
 
+// ------------------------------------------- linears on fp16 planes
+
+// An operand's planes (split_gemm.hip): `rows` rows of k elements.
+struct Planes {
+  unsigned char *p = nullptr;
+  int *exps = nullptr;
+  size_t rows = 0, k = 0;
+  size_t half = 0;  // > 0: GeGLU weights of 2 * half rows, 16-row blocks alternating
+  size_t blocks() const {
+    return half ? 2 * tfd::split_blocks(half) : tfd::split_blocks(rows);
+  }
+  size_t bytes() const { return blocks() * ((k + 31) / 32) * tfd::kSplitBlock; }
+  size_t total() const { return ((bytes() + 255) & ~(size_t)255) + ((64 * blocks() + 255) & ~(size_t)255); }
+};
+
+// Carves the planes of several operands out of c->planes.
+int reserve_planes(tfd_ctx *c, std::initializer_list<Planes *> list) {
+  size_t total = 0;
+  for (const Planes *p : list) total += p->total();
+  int rc = reserve(c, c->planes, total);
+  if (rc) return rc;
+  unsigned char *at = static_cast<unsigned char *>(c->planes.ptr);
+  for (Planes *p : list) {
+    p->p = at;
+    p->exps = reinterpret_cast<int *>(at + ((p->bytes() + 255) & ~(size_t)255));
+    at += p->total();
+  }
+  return TFD_OK;
+}
+
+bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+// The split of one operand: row r of the planes is source row map ? map[r] : r.
+// length > 0: the source is token-contiguous, (length, k) per question row.
+tfd::SplitSeg split_seg(const Planes &d, const float *src, const int *map = nullptr,
+                        size_t length = 0) {
+  tfd::SplitSeg g{};
+  g.src = src;
+  g.map = map;
+  g.dst = d.p;
+  g.exps = d.exps;
+  g.rows = (int)d.rows;
+  g.k = (int)d.k;
+  g.blocks = (int)d.blocks();
+  g.length = (int)length;
+  g.half = (int)d.half;
+  g.trans = length > 0;
+  g.vec = !g.trans && d.k % 4 == 0 && aligned16(src);
+  return g;
+}
+
+int split_rows(tfd_ctx *c, std::initializer_list<tfd::SplitSeg> list) {
+  tfd::SplitSegs segs;
+  for (const tfd::SplitSeg &g : list) segs.seg[segs.n++] = g;
+  TFD_HIP(c, tfd::launch_split_rows(segs, c->stream), "split_rows launch");
+  return TFD_OK;
+}
+
+// Whether a linear of `cols` columns (weights out x in) runs as fp16 planes:
+// from the size where splitting both operands on each call (5 us or more) plus the
+// three fp16 products undercut one f32 product, and a size the planes'
+// 32-bit indices hold.
+bool split_pays(size_t out, size_t in, size_t cols) {
+  return in >= 256 && out >= 256 && cols >= 512 && out * cols >= ((size_t)1 << 19) &&
+         in <= 65536 && out <= ((size_t)1 << 26) && cols <= ((size_t)1 << 26);
+}
+
+tfd::SplitGemmArgs split_args(const Planes &a, const Planes &b, size_t m) {
+  tfd::SplitGemmArgs g{};
+  g.a = a.p;
+  g.b = b.p;
+  g.ea = a.exps;
+  g.eb = b.exps;
+  g.m = (int)m;
+  g.n = (int)b.rows;
+  g.nkb = (int)((a.k + 31) / 32);
+  g.mrows = (int)(a.half ? 16 * a.blocks() : a.rows);
+  return g;
+}
+
+// out[:, map ? map[n] : n] (+)= W^T x (+ bias), activation: w the (in, out)
+// weight's planes, x the columns'; GeGLU when w's halves alternate.
+int split_linear(tfd_ctx *c, const Planes &w, const Planes &x, float *out, const float *bias,
+                 int act, bool accumulate = false, const int *map = nullptr) {
+  const size_t m = w.half ? w.half : w.rows;
+  tfd::SplitGemmArgs g = split_args(w, x, m);
+  g.out = out;
+  g.ldc = m;
+  g.map = map;
+  g.bias = bias;
+  g.act = act;
+  g.accumulate = accumulate ? 1 : 0;
+  g.vec = m % 4 == 0 && aligned16(out) && (!bias || aligned16(bias)) ? 1 : 0;
+  TFD_HIP(c,
+          tfd::launch_split_gemm(g, w.half ? tfd::kEpiGeglu : tfd::kEpiCols, c->cus, c->stream),
+          "split_gemm launch");
+  return TFD_OK;
+}
+
 // attention_block_tenferro (laya-infer model.rs:1304-1347) on device
 // pointers: qkv = W_in^T x (+ b_in), the fused op under a keep tensor or a
 // structured (valid, window) mask, out = W_out^T attended (+ b_out); with
@@ -665,6 +766,22 @@ int laya_layer_dev(tfd_ctx *c, const char *op, const float *x, size_t hidden, si
   // Workspace: qkv (3d, L, B), then the attention output (d, L, B).
   if ((rc = reserve(c, c->layer, sizeof(float) * 4 * n))) return rc;
   float *qkv = static_cast<float *>(c->layer.ptr), *att = qkv + 3 * n;
+  if (split_pays(hidden, hidden, tokens)) {
+    Planes wi, wo, xp;
+    wi.rows = 3 * hidden;
+    wo.rows = hidden;
+    xp.rows = tokens;
+    wi.k = wo.k = xp.k = hidden;
+    // The attention output's planes take the place of x's.
+    if ((rc = reserve_planes(c, {&wi, &wo, &xp}))) return rc;
+    if ((rc = split_rows(c, {split_seg(xp, x), split_seg(wi, w_in), split_seg(wo, w_out)})) ||
+        (rc = split_linear(c, wi, xp, qkv, b_in, tfd::kActNone)) ||
+        (rc = laya_run(c, op, qkv, keep, valid, window, hidden, heads, length, batch, rope_bits,
+                       att, TFD_DEVICE_PTRS | TFD_ASYNC)) ||
+        (rc = split_rows(c, {split_seg(xp, att)})))
+      return rc;
+    return split_linear(c, wo, xp, out, b_out, tfd::kActNone, accumulate);
+  }
   // qkv = W_in^T x (+ b_in): linear_feature_first (model.rs:1179-1216).
   if ((rc = gemm(c, true, false, 3 * hidden, tokens, hidden, w_in, hidden, 0, x, hidden, 0, qkv,
                  3 * hidden, 0, 1)))
@@ -762,6 +879,57 @@ int jeff_layer(tfd_ctx *c, size_t rows, size_t length, size_t hidden, size_t hea
   float *q = static_cast<float *>(c->layer.ptr), *g = q + qn, *merged = g + qn, *k = merged + qn,
         *v = k + kvn;
   const float *xf = static_cast<const float *>(x_d);
+  auto attend = [&] {
+    return jeff_run(c, op, false, rows, length, heads, kv_heads, head_dim, rotary_dim, q, k, v, g,
+                    static_cast<const float *>(qn_d), static_cast<const float *>(kn_d),
+                    static_cast<const float *>(m_d), theta_bits, eps_bits, merged,
+                    (flags & TFD_TRIM_LEADING) | TFD_DEVICE_PTRS | TFD_ASYNC);
+  };
+  const size_t tokens = rows * length;
+  if (split_pays(W, hidden, tokens) && split_pays(hidden, W, tokens)) {
+    // One product for the four projections: their weights' planes follow one
+    // another (each padded to whole 16-row blocks), tokens are the rows.
+    auto pad = [](size_t n) { return 16 * tfd::split_blocks(n); };
+    Planes xp, wp, wo, mp;
+    xp.rows = mp.rows = tokens;
+    xp.k = wp.k = hidden;
+    wp.rows = 2 * pad(W) + 2 * pad(KW);
+    wo.rows = hidden;
+    wo.k = mp.k = W;
+    if ((rc = reserve_planes(c, {&xp, &wp, &wo, &mp}))) return rc;
+    const float *w4[4] = {static_cast<const float *>(wq_d), static_cast<const float *>(wg_d),
+                          static_cast<const float *>(wk_d), static_cast<const float *>(wv_d)};
+    float *y4[4] = {q, g, k, v};
+    const size_t n4[4] = {W, W, KW, KW};
+    tfd::SplitGemmArgs ga = split_args(xp, wp, tokens);
+    tfd::SplitSeg s4[4];
+    size_t at = 0;
+    for (int i = 0; i < 4; ++i) {
+      Planes part = wp;
+      part.rows = n4[i];
+      part.p = wp.p + at / 16 * ((hidden + 31) / 32) * tfd::kSplitBlock;
+      part.exps = wp.exps + at;
+      s4[i] = split_seg(part, w4[i]);
+      ga.outs[i] = tfd::SplitOut{y4[i], (int)at, (int)n4[i]};
+      at += pad(n4[i]);
+    }
+    ga.nouts = 4;
+    ga.length = (int)length;
+    ga.vec = length % 4 == 0 && qn % 4 == 0 && kvn % 4 == 0 ? 1 : 0;
+    if ((rc = split_rows(c, {split_seg(xp, xf, nullptr, length), s4[0], s4[1], s4[2], s4[3],
+                             split_seg(wo, static_cast<const float *>(wo_d))})))
+      return rc;
+    TFD_HIP(c, tfd::launch_split_gemm(ga, tfd::kEpiRows, c->cus, c->stream), "split_gemm launch");
+    if ((rc = attend()) || (rc = split_rows(c, {split_seg(mp, merged, nullptr, length)})))
+      return rc;
+    tfd::SplitGemmArgs go = split_args(mp, wo, tokens);
+    go.outs[0] = tfd::SplitOut{static_cast<float *>(out_d), 0, (int)hidden};
+    go.nouts = 1;
+    go.length = (int)length;
+    go.vec = length % 4 == 0 && aligned16(out_d) ? 1 : 0;
+    TFD_HIP(c, tfd::launch_split_gemm(go, tfd::kEpiRows, c->cus, c->stream), "split_gemm launch");
+    return finish(c, flags, out, out_d, sizeof(float) * xn);
+  }
   // y_r = x_r W for every row r, (L, hidden) x (hidden, out): linear_tenferro
   // (model.rs:289-317).
   auto proj = [&](const void *w, size_t out_dim, float *y) {
@@ -771,11 +939,7 @@ int jeff_layer(tfd_ctx *c, size_t rows, size_t length, size_t hidden, size_t hea
   if ((rc = proj(wq_d, W, q)) || (rc = proj(wg_d, W, g)) || (rc = proj(wk_d, KW, k)) ||
       (rc = proj(wv_d, KW, v)))
     return rc;
-  if ((rc = jeff_run(c, op, false, rows, length, heads, kv_heads, head_dim, rotary_dim, q, k, v, g,
-                     static_cast<const float *>(qn_d), static_cast<const float *>(kn_d),
-                     static_cast<const float *>(m_d), theta_bits, eps_bits, merged,
-                     (flags & TFD_TRIM_LEADING) | TFD_DEVICE_PTRS | TFD_ASYNC)))
-    return rc;
+  if ((rc = attend())) return rc;
   if ((rc = gemm(c, false, false, length, hidden, W, merged, length, length * W,
                  static_cast<const float *>(wo_d), W, 0, static_cast<float *>(out_d), length,
                  length * hidden, rows)))
@@ -986,6 +1150,45 @@ int laya_forward(tfd_ctx *c, const tfd_laya_model *m, const int64_t *ids, const 
         *a1 = take(AH * B);
   const bool dev_out = (flags & TFD_DEVICE_PTRS) != 0;
   float *act_d = dev_out ? action : take(A * B), *log_d = dev_out ? logits : take(KB);
+  // Long batches: the layers' linears on fp16 planes, split layer by layer.
+  // Columns that are normalized first are written as planes by the norm.
+  const bool split = split_pays(d, d, Tc) && (m->n_layers == 0 || split_pays(d, I, Tc)) &&
+                     tfd::norm_split_fits((int)d);
+  Planes p_qkv, p_wo, p_wi, p_wm, p_x, p_g;  // weights, d-wide columns, wider columns
+  if (split) {
+    p_qkv.rows = 3 * d;
+    p_wo.rows = p_wm.rows = d;
+    p_qkv.k = p_wo.k = p_wi.k = p_x.k = d;
+    p_wi.rows = std::max(2 * I, ff_max);
+    p_wi.half = 0;
+    p_wm.k = p_g.k = std::max(I, ff_max);
+    p_x.rows = p_g.rows = Tc;
+    if (m->n_layers) p_wi.rows += 32;  // each GeGLU half is padded to whole blocks
+    if ((rc = reserve_planes(c, {&p_qkv, &p_wo, &p_wi, &p_wm, &p_x, &p_g}))) return rc;
+  }
+  auto norm_planes = [&](const float *in, const float *w, const float *b) {
+    tfd::NormArgs na{};
+    na.x = in;
+    na.w = w;
+    na.b = b;
+    na.cols = (long)Tc;
+    na.ldx = na.d = (int)d;
+    na.per = 1;
+    na.eps = eps;
+    TFD_HIP(c, tfd::launch_norm_split(na, p_x.p, p_x.exps, c->stream), "norm launch");
+    return (int)TFD_OK;
+  };
+  // The attention block on p_x's columns with p_qkv and p_wo, added into res.
+  auto split_attention = [&](size_t heads, int64_t window, const float *b_in, const float *b_out,
+                             uint32_t rope_bits, float *res) {
+    int r = split_linear(c, p_qkv, p_x, qkv_f, b_in, tfd::kActNone, false, d_cols);
+    if (r) return r;
+    if ((r = laya_run(c, op, qkv_f, nullptr, d_valid, window, d, heads, L, B, rope_bits, att_f,
+                      TFD_DEVICE_PTRS | TFD_ASYNC, d_need)))
+      return r;
+    if ((r = split_rows(c, {split_seg(p_x, att_f, d_cols)}))) return r;
+    return split_linear(c, p_wo, p_x, res, b_out, tfd::kActNone, true);
+  };
   // Padded columns of the attention input that no packed column fills stay 0.
   TFD_HIP(c, tfd::launch_fill_zero(qkv_f, 3 * xs, c->stream), "fill launch");
 
@@ -1016,6 +1219,26 @@ int laya_forward(tfd_ctx *c, const tfd_laya_model *m, const int64_t *ids, const 
     return rc;
   for (size_t i = 0; i < m->n_layers; ++i) {
     const tfd_laya_encoder_layer &l = m->layers[i];
+    if (split) {
+      Planes wi = p_wi, wm = p_wm, gp = p_g;
+      wi.rows = 2 * I;
+      wi.half = I;
+      wm.k = gp.k = I;
+      if ((rc = split_rows(c, {split_seg(p_qkv, l.wqkv), split_seg(p_wo, l.wo),
+                               split_seg(wi, l.wi), split_seg(wm, l.wo_mlp)})))
+        return rc;
+      rc = l.attn_norm_w ? norm_planes(x, l.attn_norm_w, l.attn_norm_b)
+                         : split_rows(c, {split_seg(p_x, x)});
+      if (rc ||
+          (rc = split_attention(m->heads, l.sliding ? (int64_t)m->window : -1, l.bqkv, l.bo,
+                                l.rope_base_bits, x)) ||
+          (rc = norm_planes(x, l.mlp_norm_w, l.mlp_norm_b)) ||
+          (rc = split_linear(c, wi, p_x, g, l.bi, tfd::kActNone)) ||
+          (rc = split_rows(c, {split_seg(gp, g)})) ||
+          (rc = split_linear(c, wm, gp, x, l.bo_mlp, tfd::kActNone, true)))
+        return rc;
+      continue;
+    }
     const float *ain = x;
     if (l.attn_norm_w) {
       if ((rc = norm_cols(c, x, nullptr, (long)Tc, d, l.attn_norm_w, l.attn_norm_b, eps, a)))
@@ -1040,6 +1263,20 @@ int laya_forward(tfd_ctx *c, const tfd_laya_model *m, const int64_t *ids, const 
   // Head layers, full attention without RoPE (model.rs:715-747, 932-935).
   for (size_t i = 0; i < m->n_head_layers; ++i) {
     const tfd_laya_head_layer &hl = m->head[i];
+    if (split) {
+      Planes w1 = p_wi, w2 = p_wm, up = p_g;
+      w1.rows = w2.k = up.k = hl.ff;
+      if ((rc = split_rows(c, {split_seg(p_qkv, hl.in_proj_w), split_seg(p_wo, hl.out_proj_w),
+                               split_seg(w1, hl.linear1_w), split_seg(w2, hl.linear2_w)})) ||
+          (rc = norm_planes(h, hl.norm1_w, hl.norm1_b)) ||
+          (rc = split_attention(hl.heads, -1, hl.in_proj_b, hl.out_proj_b, 0u, h)) ||
+          (rc = norm_planes(h, hl.norm2_w, hl.norm2_b)) ||
+          (rc = split_linear(c, w1, p_x, u, hl.linear1_b, tfd::kActRelu)) ||
+          (rc = split_rows(c, {split_seg(up, u)})) ||
+          (rc = split_linear(c, w2, up, h, hl.linear2_b, tfd::kActNone, true)))
+        return rc;
+      continue;
+    }
     if ((rc = norm_cols(c, h, nullptr, (long)Tc, d, hl.norm1_w, hl.norm1_b, eps, n))) return rc;
     if ((rc = attention(n, hl.heads, -1, hl.in_proj_w, hl.in_proj_b, hl.out_proj_w, hl.out_proj_b,
                         0u, h)))
@@ -1124,6 +1361,7 @@ void tfd_ctx_destroy(tfd_ctx *c) {
     if (c->bits.ptr) (void)hipFree(c->bits.ptr);
     if (c->kp.ptr) (void)hipFree(c->kp.ptr);
     if (c->layer.ptr) (void)hipFree(c->layer.ptr);
+    if (c->planes.ptr) (void)hipFree(c->planes.ptr);
     if (c->model.ptr) (void)hipFree(c->model.ptr);
     if (c->blas) (void)rocblas_destroy_handle(c->blas);
     for (auto &e : c->rope) {
@@ -1154,7 +1392,7 @@ void *tfd_ctx_stream(tfd_ctx *c) {
 
 size_t tfd_ctx_retained_bytes(const tfd_ctx *c) {
   if (!c) return 0;
-  size_t total = sizeof(tfd_ctx) + c->bits.cap + c->kp.cap + c->layer.cap + c->model.cap +
+  size_t total = sizeof(tfd_ctx) + c->bits.cap + c->kp.cap + c->layer.cap + c->model.cap + c->planes.cap +
                  c->model_host.capacity();
   for (const auto &b : c->staging) total += b.cap;
   for (const auto &e : c->rope) total += e.bytes;

@@ -243,4 +243,62 @@ hipError_t launch_pool(const PoolArgs &a, int batch, hipStream_t stream);
 hipError_t launch_copy_columns(const float *src, const int *src_map, float *dst,
                                const int *dst_map, int m, long n, hipStream_t stream);
 
+// ------------------------------------------------ f32 linears on fp16 planes
+
+// Bytes of one plane block: 16 rows x 32 k, hi then lo (split_gemm.hip).
+constexpr int kSplitBlock = 2048;
+inline size_t split_blocks(size_t rows) { return (rows + 15) / 16; }
+inline size_t split_plane_bytes(size_t rows, size_t k) {
+  return split_blocks(rows) * ((k + 31) / 32) * kSplitBlock;
+}
+
+// One operand to split: `blocks` plane row blocks of k elements each.
+struct SplitSeg {
+  const float *src;
+  const int *map;      // or null: plane row p reads source row map[p]
+  unsigned char *dst;  // split_plane_bytes
+  int *exps;           // 16 * blocks
+  int rows, k, blocks;
+  int length;          // trans: tokens per question row
+  int half;            // > 0: alternate 16-row blocks of rows 0.. and half.. (GeGLU)
+  bool trans;          // source (length, k) per question row, token-contiguous
+  bool vec;            // 16-byte aligned rows, k % 4 == 0, not trans
+};
+constexpr int kSplitSegs = 6;
+struct SplitSegs {
+  SplitSeg seg[kSplitSegs];
+  int n = 0;
+};
+hipError_t launch_split_rows(const SplitSegs &segs, hipStream_t stream);
+
+enum SplitEpilogue : int {
+  kEpiCols = 0,   // out[m + ldc * (map ? map[n] : n)] (+)= A_m . B_n (+ bias[m]), activation
+  kEpiGeglu = 1,  // out[f + ldc * n] = gelu(first half) * second half (A interleaved, SplitSeg::half)
+  kEpiRows = 2,   // rows of A are tokens of question rows, columns features of `outs`
+};
+struct SplitOut {
+  float *ptr;        // rows x (length, width)
+  int begin, width;  // its first column of B, its features
+};
+struct SplitGemmArgs {
+  const unsigned char *a, *b;  // planes
+  const int *ea, *eb;
+  int m, n, nkb;     // outputs along A (kEpiGeglu: one half's), columns, 32-k blocks
+  int mrows;         // plane rows of A (kEpiGeglu: both halves, padded to 16)
+  int mt, nt;        // tiles (set by the launcher)
+  float *out;
+  size_t ldc;
+  const int *map;    // output column of column n, or null
+  const float *bias;
+  int act, accumulate;
+  int vec;           // bit 0: 16-byte stores allowed
+  SplitOut outs[4];
+  int nouts, length;
+};
+hipError_t launch_split_gemm(const SplitGemmArgs &g, int epi, int cus, hipStream_t stream);
+// LayerNorm (a.y, a.add unused) straight into planes; d as norm_split_fits says.
+bool norm_split_fits(int d);
+hipError_t launch_norm_split(const NormArgs &a, unsigned char *dst, int *exps,
+                             hipStream_t stream);
+
 }  // namespace tfd

@@ -26,6 +26,7 @@ HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 KERNELS = [
     ("jeff_bf16_wide.hip", "_ZN3tfd21jeff_bf16_wide_kernel"),
     ("jeff_attention.hip", "_ZN3tfd21jeff_split_f32_kernelILi256E"),
+    ("split_gemm.hip", "_ZN3tfd12_GLOBAL__N_117split_gemm_kernelILi128ELi128E"),
 ]
 
 
