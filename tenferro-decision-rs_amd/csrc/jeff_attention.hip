@@ -115,18 +115,6 @@ __device__ __forceinline__ void wave_active_span(const float *maskr, int L, int 
   last = __builtin_amdgcn_readfirstlane(hi);
 }
 
-// Split layout (f32, HDP = 256, for the split-head kernel): each (row, kv
-// head) holds Lp = L rounded up to 16 keys, as blocks of 16 keys x 64
-// features (tile kt, wave slice w) of 4 KB, each four 1 KB runs c: run c,
-// 16-byte chunk 16g + col is key 16kt + col, features 64w + 16c + 4g .. + 3.
-// A wave's load of run c is then one contiguous 1 KB read. Keys L .. Lp - 1
-// hold zeros.
-__device__ __forceinline__ size_t split_kp_offset(int key, int d) {
-  const int kt = key >> 4, col = key & 15;
-  const int w = d >> 6, c = (d >> 4) & 3, g = (d >> 2) & 3, e = d & 3;
-  return ((size_t)(kt * 4 + w) * 4 + c) * 256 + (g * 16 + col) * 4 + e;
-}
-
 // One wavefront: the row's active keys (mask != 0) as one bit per key (zero
 // past L, 32 keys per word) and its (first, last) span, (0, -1) for a row
 // with none, for the attention kernels' scalar loads.
@@ -292,54 +280,101 @@ __global__ __launch_bounds__(256) void jeff_k_prep_kernel(const JeffArgs a, OutT
   }
 }
 
-// K prep for the split-head kernel (f32, HDP = 256): one workgroup = 32 keys
-// (two 16-key tiles) of one (row, kv head), written in the split layout
-// above. K arrives along keys as whole 128-byte rows (feature d, keys
-// k0 .. k0 + 31: eight 16-byte loads per feature, eight per thread) and is
-// transposed through LDS; thread (key tid & 31, part tid >> 5) then owns
-// features 32 part .. + 31 of its key: RMSNorm (lib.rs:676-691) with the
-// sum of squares reduced over the eight parts (lane swap, then LDS),
-// partial RoPE (692-709) in registers when the partner feature i + rot/2
-// sits in the same wave (rot/2 = 32: part p pairs with part p + 1, lane
-// + 32), else through LDS. Workgroups with blockIdx.x == 0 and kv head 0
-// also write the row's active-key bits and key span.
-__global__ __launch_bounds__(256) void jeff_k_prep_split_kernel(const JeffArgs a,
-                                                                float *__restrict__ kp,
-                                                                int *__restrict__ spans,
-                                                                uint32_t *__restrict__ kbits) {
+// Planes of the f32 kernel at hd 256: per (row, kv head) and 32-key tile 64
+// KB in the order the 16x16x32 fp16 matrix cores read them, every f32 as hi +
+// lo fp16 (1 KB blocks, 16 bytes per lane, hi then lo). K: blocks (16-key half
+// b, step s), lane (key, g) holding features 32 s + 8 g .. + 7. V: blocks of 16
+// features, lane (feature, g) holding keys 4 g .. + 3 and 16 + 4 g .. + 3, the
+// keys whose probabilities lane group g of S^T holds.
+constexpr int kJeffTileBytes = 65536, kJeffTileV = 32768;
+// Normalized keys and queries times 2^(kJeffNormUp - e), e =
+// norm_weight_exp: below 2^14, so lo still holds elements 2^-24 of the largest
+// to 2^-11 of themselves.
+constexpr int kJeffNormUp = 10;
+
+// One workgroup = the K (blockIdx.y even) or V planes of one (row, kv head,
+// 32-key tile): the split done once per call instead of once per query tile
+// that reads the tile (16 or more at L 256). K: thread (key tid & 31, part
+// tid >> 5) owns features 32 part .. + 31 of its key, loaded with one 128-byte
+// run per feature; RMSNorm (lib.rs:676-691) with the sum of squares reduced
+// over the eight parts (lane swap, then LDS), partial RoPE (692-709) in
+// registers when the partner feature i + rot/2 sits in the same wave (rot/2 =
+// 32: part p pairs with part p + 1, lane + 32), else through LDS. V: thread =
+// feature, its 32 keys as eight 16-byte loads (dword alignment suffices),
+// scaled by 2^-e of the tile's largest magnitude (vexp). Workgroups with
+// blockIdx.x == 0 of kv head 0 also write the row's active-key bits and key
+// span, row 0's the norm exponents (spans[-2], spans[-1]). Bound by HBM and one
+// memory round trip.
+__global__ __launch_bounds__(256) void jeff_k_prep_split_kernel(
+    const JeffArgs a, unsigned char *__restrict__ planes, int *__restrict__ vexp,
+    int *__restrict__ spans, uint32_t *__restrict__ kbits) {
   constexpr int HDP = 256, KB = 32, KS = HDP + 4;
   __shared__ __attribute__((aligned(16))) float Kt[KB * KS];
   __shared__ float s_red[4 * KB];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int row = blockIdx.z, kvh = blockIdx.y;
+  const int row = blockIdx.z, kvh = blockIdx.y >> 1;
+  const bool is_v = (blockIdx.y & 1) != 0;
   const int L = a.L, hd = a.hd, rh = a.rot_half;
   const int k0 = blockIdx.x * KB;
   const float *maskr = a.mask + (size_t)row * L;
-  const float *K = static_cast<const float *>(a.k) + row * a.kv_row + (size_t)kvh * a.kv_head;
 
-  // A block with no active key is never read: the attention kernel walks
-  // only from the row's first active key on, and inside that range it skips
-  // (or masks whole) tiles without active keys. Such blocks leave their
-  // workspace untouched, except the one that also writes the row's bits.
-  if (!(blockIdx.x == 0 && kvh == 0)) {
+  // A tile with no active key is never read by a wave that computes with it.
+  // Such blocks leave their workspace untouched, except the one that also
+  // writes the row's bits.
+  if (!(blockIdx.x == 0 && blockIdx.y == 0)) {
     const int kl = min(k0 + (lane & 31), L - 1);
     const bool act = k0 + (lane & 31) < L && maskr[kl] != 0.0f;
     if (__ballot(act) == 0) return;  // the same in every wave
   }
+  const size_t unit = ((size_t)row * a.kv_heads + kvh) * gridDim.x + blockIdx.x;
+  unsigned char *tile = planes + unit * kJeffTileBytes;
 
-  // Raw block along keys: task (feature d, keys k0 + 4 g8 .. + 3), L % 4 == 0;
-  // features past hd and keys past L read as 0 (keys past L of this feature
-  // are the next feature's and are zeroed below).
-  const __amdgpu_buffer_rsrc_t rk = buffer_rsrc(K, (uint32_t)((size_t)hd * L * 4));
-  f32x4 x[8];
+  if (is_v) {
+    const float *V = static_cast<const float *>(a.v) + row * a.kv_row + (size_t)kvh * a.kv_head;
+    const __amdgpu_buffer_rsrc_t rv = buffer_rsrc(V, (uint32_t)((size_t)hd * L * 4));
+    f32x4 x[8];
 #pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    const int e = tid + 256 * t, d = e >> 3, g8 = e & 7;
-    x[t] = buffer_load4(rk, (d * L + 4 * g8) * 4, k0 * 4);
+    for (int c = 0; c < 8; ++c) x[c] = buffer_load4(rv, (tid * L + 4 * c) * 4, k0 * 4);
+    float mx = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        // Past L lies the next feature; past hd the loads read 0.
+        x[c][e] = k0 + 4 * c + e < L ? x[c][e] : 0.0f;
+        mx = fmaxf(mx, __builtin_isfinite(x[c][e]) ? fabsf(x[c][e]) : 0.0f);
+      }
+    mx = wave_max_f(mx);
+    if (lane == 0) s_red[wave] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
+    const int ev = max(-126, (int)(__float_as_uint(mx) >> 23) - 126 - 15);  // zero or denormal: -126
+    if (tid == 0) vexp[unit] = ev;
+    const float sc = pow2i(-ev);
+    unsigned char *p = tile + kJeffTileV + (tid >> 4) * 2048 + (tid & 15) * 16;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f16x4 h0, l0, h1, l1;
+      split_f16(x[g], sc, h0, l0);
+      split_f16(x[4 + g], sc, h1, l1);
+      *reinterpret_cast<f16x8 *>(p + 256 * g) = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+      *reinterpret_cast<f16x8 *>(p + 256 * g + 1024) =
+          __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+    return;
   }
+
+  const float *K = static_cast<const float *>(a.k) + row * a.kv_row + (size_t)kvh * a.kv_head;
+  const __amdgpu_buffer_rsrc_t rk = buffer_rsrc(K, (uint32_t)((size_t)hd * L * 4));
   const int kk = tid & 31, part = tid >> 5;  // this thread's key and 32-feature part
   const int key = k0 + kk;
   const bool kin = key < L;
+  float kv[32];
+  {
+    const int off = (32 * part * L + key) * 4;  // features past hd read as 0
+#pragma unroll
+    for (int i = 0; i < 32; ++i) kv[i] = buffer_load1(rk, off, i * L * 4);
+  }
   const __amdgpu_buffer_rsrc_t rn = buffer_rsrc(a.k_norm, (uint32_t)(hd * 4));
   f32x4 wn[8];
 #pragma unroll
@@ -355,26 +390,23 @@ __global__ __launch_bounds__(256) void jeff_k_prep_split_kernel(const JeffArgs a
       ts[c] = *reinterpret_cast<const f32x4 *>(a.sin_t + pos + 4 * c);
     }
   }
-
-  if (blockIdx.x == 0 && kvh == 0 && wave == 0) write_row_bits_span(maskr, L, lane, row, spans, kbits);
-
-#pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    const int e = tid + 256 * t, d = e >> 3, g8 = e & 7;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) Kt[(4 * g8 + i) * KS + d] = x[t][i];
+  const int ek = norm_weight_exp(a.k_norm, hd, lane);
+  if (blockIdx.x == 0 && kvh == 0 && wave == 0) {
+    write_row_bits_span(maskr, L, lane, row, spans, kbits);
+    if (row == 0) {  // the attention kernel's norm exponents
+      const int eq = norm_weight_exp(a.q_norm, hd, lane);
+      if (lane == 0) {
+        spans[-2] = eq;
+        spans[-1] = ek;
+      }
+    }
   }
-  __syncthreads();
-  float kv[32];
+
   float ss = 0.0f;
 #pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const f32x4 y = *reinterpret_cast<const f32x4 *>(&Kt[kk * KS + 32 * part + 4 * c]);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      kv[4 * c + e] = kin ? y[e] : 0.0f;
-      ss += kv[4 * c + e] * kv[4 * c + e];
-    }
+  for (int i = 0; i < 32; ++i) {
+    kv[i] = kin ? kv[i] : 0.0f;  // past L lies the next feature
+    ss += kv[i] * kv[i];
   }
   ss = pair_sum(ss);  // the wave's two parts of this key
   if (lane < 32) s_red[wave * KB + lane] = ss;
@@ -403,7 +435,6 @@ __global__ __launch_bounds__(256) void jeff_k_prep_split_kernel(const JeffArgs a
       }
     }
   } else if (rope) {
-    __syncthreads();
 #pragma unroll
     for (int j = 0; j < 32; ++j) Kt[kk * KS + 32 * part + j] = kv[j];
     __syncthreads();
@@ -419,14 +450,15 @@ __global__ __launch_bounds__(256) void jeff_k_prep_split_kernel(const JeffArgs a
 #pragma unroll
     for (int j = 0; j < 32; ++j) kv[j] = Kt[kk * KS + 32 * part + j];
   }
-  const int Lp = (L + 15) & ~15;
-  if (key < Lp) {
-    float *unit = kp + ((size_t)row * a.kv_heads + kvh) * (size_t)Lp * HDP;
+  const float sc = pow2i(kJeffNormUp - ek);
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const f32x4 o = {kv[4 * c], kv[4 * c + 1], kv[4 * c + 2], kv[4 * c + 3]};
-      *reinterpret_cast<f32x4 *>(unit + split_kp_offset(key, 32 * part + 4 * c)) = o;
-    }
+  for (int c = 0; c < 4; ++c) {  // step part, lane group c
+    f16x4 h0, l0, h1, l1;
+    split_f16(f32x4{kv[8 * c], kv[8 * c + 1], kv[8 * c + 2], kv[8 * c + 3]}, sc, h0, l0);
+    split_f16(f32x4{kv[8 * c + 4], kv[8 * c + 5], kv[8 * c + 6], kv[8 * c + 7]}, sc, h1, l1);
+    unsigned char *p = tile + ((kk >> 4) * 8 + part) * 2048 + (c * 16 + (kk & 15)) * 16;
+    *reinterpret_cast<f16x8 *>(p) = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+    *reinterpret_cast<f16x8 *>(p + 1024) = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
   }
 }
 
@@ -600,15 +632,23 @@ __device__ __forceinline__ void jeff_store(const JeffArgs &a, const float *Gt, f
 #pragma unroll
       for (int u = 0; u < NG; ++u) {
         const int e = min(i0 + lane + 64 * u, HDP * 4 - 1), d = e >> 2, gq = e & 3;
-        const int qa = q0 + 4 * gq;  // L % 4 == 0: the 4 queries are all in or all out
+        const int qa = q0 + 4 * gq;
         f32x4 o;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           const float x = ow[(4 * gq + t) * QP + d] * fast_sigmoid(g[u][t]);
           o[t] = qa + t < start ? 0.0f : x;
         }
-        if (qa < L && d < hd && d >= d_lo && d < d_hi)
-          buffer_store4_nt(o, ro, (int)(((size_t)d * L + 4 * gq) * 4), q0 * 4);
+        if (d < hd && d >= d_lo && d < d_hi) {
+          const int off = (int)(((size_t)d * L + 4 * gq) * 4);
+          if (qa + 4 <= L) {
+            buffer_store4_nt(o, ro, off, q0 * 4);
+          } else {  // the row ends inside these four queries (L % 4 != 0) or before them
+#pragma unroll
+            for (int t = 0; t < 3; ++t)
+              if (qa + t < L) buffer_store1_nt(o[t], ro, off + 4 * t, q0 * 4);
+          }
+        }
       }
     }
   } else {
@@ -711,9 +751,8 @@ struct JeffStage {
 };
 
 // TAG gives each calling kernel its own copy, compiled to that kernel's
-// register budget; TAG 1 (the split-head kernel) reads the split K layout,
-// TAG 2 (the fused kernel, no K prep) normalizes and rotates each key tile
-// from K itself into LDS.
+// register budget; TAG 1 (the split kernel) and TAG 2 (the fused kernels)
+// normalize and rotate each key tile from K itself into LDS.
 template <int HDP, bool VEC, int TAG = 0>
 __device__ __noinline__ void jeff_redo_wave(const JeffArgs *ap, const float *__restrict__ kp,
                                             int row, int head, int q0, int kt_begin, int kt_end,
@@ -966,10 +1005,8 @@ __device__ __noinline__ void jeff_redo_wave(const JeffArgs *ap, const float *__r
   const float *Q = static_cast<const float *>(a.q) + row * a.q_row + (size_t)head * hd * L;
   const float *Gt = static_cast<const float *>(a.gate) + row * a.q_row + (size_t)head * hd * L;
   const float *V = static_cast<const float *>(a.v) + row * a.kv_row + (size_t)kvh * a.kv_head;
-  constexpr bool SPLIT = TAG == 1;
-  constexpr bool RAW = TAG == 2;  // keys straight from K, normalized per tile into LDS
-  const size_t Lu = SPLIT ? (size_t)((L + 15) & ~15) : (size_t)L;
-  const float *KP = RAW ? nullptr : kp + ((size_t)row * a.kv_heads + kvh) * Lu * HDP;
+  constexpr bool RAW = TAG != 0;  // keys straight from K, normalized per tile into LDS
+  const float *KP = RAW ? nullptr : kp + ((size_t)row * a.kv_heads + kvh) * (size_t)L * HDP;
   const float *Kraw = static_cast<const float *>(a.k) + row * a.kv_row + (size_t)kvh * a.kv_head;
   constexpr int QP = HDP + 4;
   float *Kw = ws + 512;  // RAW: 16 keys x QP floats, after Pw
@@ -1034,8 +1071,7 @@ __device__ __noinline__ void jeff_redo_wave(const JeffArgs *ap, const float *__r
     for (int r = 0; r < 4; ++r) s[r] = 0.0f;
 #pragma unroll
     for (int x = 0; x < QS; ++x) {
-      const float kx = SPLIT ? KP[split_kp_offset(kcl, grp * QS + x)] : krow[x];  // RAW: LDS
-      s = mfma_16x16x4(kc < L ? kx : 0.0f, qreg[x], s);
+      s = mfma_16x16x4(kc < L ? krow[x] : 0.0f, qreg[x], s);
     }
     float mx = -INFINITY;
 #pragma unroll
@@ -1095,7 +1131,7 @@ __device__ __noinline__ void jeff_redo_wave(const JeffArgs *ap, const float *__r
 
 // ------------------------------------------------- f32 attention, split head
 
-// (row, head) of work unit u < rows * heads of the split-head and fused
+// (row, head) of work unit u < rows * heads of the fused
 // kernels, whose grids are (units, query tiles) and dispatch in the linear
 // order u + units * y, workgroup id % 8 being the XCD: when the counts allow
 // it, the 8 * G consecutive units of one XCD round are the G query heads of
@@ -1117,476 +1153,359 @@ __device__ __forceinline__ void jeff_unit_of(const JeffArgs &a, int rows, int u,
   }
 }
 
-// One workgroup = 4 wavefronts = one (row, head, 16-query tile). Wave w owns
-// features [w*DS, (w+1)*DS) of the head (DS = HDP/4 = 64) in both products:
-//   S^T_w (16 keys x 16 queries) = K[keys, slice w] Q[queries, slice w]^T  (16 MFMA 16x16x4)
-//   S^T = sum over w of S^T_w, exchanged through LDS, one barrier per tile
-//   O^T[slice w] += V[slice w]^T P^T                                       (16 MFMA 16x16x4)
-// so a query tile's key walk runs on four SIMDs at once, and the longest
-// tiles (the last query tiles of full rows) no longer bound the kernel.
-// Every wave holds the same scores and runs the same softmax, so all control
-// flow is workgroup-uniform.
-//
-// Memory: K comes from the prep workspace in the split layout (each wave's
-// run of a tile is one contiguous 1 KB read), V columns straight from V;
-// the next tile's K and V slices go into the wave's LDS with LDS-DMA loads
-// while the current tile is computed, so no second tile of registers is
-// held: the kernel fits 128 VGPRs, four workgroups per CU. Q, the gate and
-// the output move along tokens
-// 16 bytes at a time and are transposed in the wave's own LDS rows, so a
-// wave issues four vector memory instructions per tensor. The row's key span
-// and active-key bits come from the prep (scalar loads).
+// One workgroup = 4 wavefronts = hg query heads of a GQA group (hg = 4, 2 or
+// 1) x 4 / hg query tiles of 16; a wave owns one head's 16 queries and walks
+// the group's 32-key tiles with every f32 product as three fp16 ones
+// (hi*hi + hi*lo + lo*hi, f32 accumulation):
+//   S^T (2 x 16 keys x 16 queries) = K_tile Q^T     (48 MFMA 16x16x32)
+//   O^T (256 x 16)                += V_tile^T P^T   (48 MFMA 16x16x32)
+// About 1,800 matrix-core cycles per wave and tile instead of 8,192 in f32, with
+// the vector work beside them (f32 MFMAs exclude it). Q is normalized and
+// rotated once into registers (hi + lo, 64 of them) and O^T stays there (64).
+// The tile's planes (jeff_k_prep_split_kernel) come by LDS-DMA into one K and
+// one V buffer: K of the next tile is loaded during the softmax and P.V, V
+// during the scores, so 64 KB serve a workgroup and two of them share a CU:
+// one's loads of Q (a burst of the whole tensor over all CUs: 4-5 us), waits and
+// output stores run beside the other's products. Two buffers of each with one
+// workgroup per CU measured 45 us against 39 at 16 rows x 256 and 49 against 46
+// at 5 x 333; eight waves sharing a tile 45. Stamps of a tile (cycles): scores
+// 1,500-1,800, softmax 500-750, P.V 1,200, waits and barriers about 450.
+// Measured with the prep: 16 rows x 256 left-padded 48-54 -> 39 us, 5 rows x 333
+// 108 -> 46 us (it ran element loads without this path).
 //
 // Workgroups are numbered from the last query tile down, so the longest
-// causal walks start first; within one query tile, the workgroups of one
-// (row, kv head) share an id residue mod 8 (one XCD, one L2) when the counts
-// allow it (jeff_unit_of).
+// causal walks start first; the workgroups of one (row, kv head) share an id
+// residue mod 8 (one XCD, one L2) when rows x kv heads is a multiple of 8.
 template <int HDP>
-__global__ __launch_bounds__(256, 4) void jeff_split_f32_kernel(const JeffArgs a,
-                                                                const float *__restrict__ kp,
-                                                                const int *__restrict__ spans,
-                                                                const uint32_t *__restrict__ kbits,
-                                                                int rows) {
-  static_assert(HDP == 256, "split-head kernel: four 64-feature slices");
-  constexpr int DS = HDP / 4;    // features per wave
-  constexpr int QS = DS / 4;     // Q registers per lane: MFMA steps per tile
-  constexpr int NB = DS / 16;    // 16-feature blocks of O^T per wave
-  constexpr int KT = kJeffKeyTile;
-  constexpr int QW = DS + 4;     // wave rows [query][feature] for Q
-  constexpr int OW = 16;         // wave rows [feature][query] for the output (the K slice)
-  constexpr int WROWS = DS * OW > 16 * QW ? DS * OW : 16 * QW;
-  constexpr int QP = HDP + 4;    // whole-tile Q rows (RoPE widths other than 16, 32)
-  constexpr int WAREA = 4 * WROWS > 16 * QP ? 4 * WROWS : 16 * QP;
-  constexpr int SX = 2 * 4 * 64 * 4;  // score exchange: 2 buffers x 4 waves x 64 lanes x f32x4
-  // Each wave's K and V tile slices (4 KB each), where the next tile lands
-  // while the current one is computed; the wave rows and the whole-tile Q
-  // rows use the same bytes before the walk and after it. 40 KB in all, so
-  // four workgroups share a CU's 160 KB.
-  constexpr int KVW = 2 * QS * 64;  // floats per wave: K and V, 16 floats per lane each
-  constexpr int KVAREA = 4 * KVW;
-  static_assert(WAREA <= KVAREA && WROWS <= KVW && DS * OW <= QS * 64,
-                "the wave rows alias the wave's tile slices; the output rows its K slice");
-  __shared__ __attribute__((aligned(16))) float smem[KVAREA + SX];
-  // RMSNorm partial sums in exchange buffer 1, read before its first use.
-  float *const s_ssq = smem + KVAREA + SX / 2;
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+__global__ __launch_bounds__(256, 2) void jeff_split_f32_kernel(
+    const JeffArgs a, const unsigned char *__restrict__ planes, const int *__restrict__ vexp,
+    const int *__restrict__ spans, const uint32_t *__restrict__ kbits, int rows) {
+  static_assert(HDP == 256, "plane layout of 64 KB tiles");
+  constexpr int NB = HDP / 16, ST = HDP / 32;
+  // Per wave: the redo's rows (512 + 16 * (HDP + 4) floats), of which the Q
+  // prep and the output use 16 * (HDP + 4). The K and V buffers alias them.
+  constexpr int WROWS = 512 + 16 * (HDP + 4);
+  constexpr int PW = 8;  // 1 KB pieces of a half tile (K or V) per wave
+  static_assert(4 * WROWS * 4 >= kJeffTileBytes, "the tile buffers alias the wave rows");
+  __shared__ __attribute__((aligned(16))) float smem[4 * WROWS];
+  unsigned char *const lds = reinterpret_cast<unsigned char *>(smem);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
-  const int L = a.L, hd = a.hd;
+  const int L = a.L, hd = a.hd, hg = a.heads_per_group;
+  float *const ws = smem + wave * WROWS;
 
-  // Issue priority (s_setprio, within this kernel's waves on a SIMD): the
-  // prologue and the epilogue above the walks of the CU's other workgroups,
-  // so that a workgroup reaches its walk, and frees its slot, sooner (f32
-  // MFMAs and vector instructions of a SIMD never run at the same time).
-  __builtin_amdgcn_s_setprio(2);
-
-  // -------- work item: query tiles from the last one down (blockIdx.y),
-  // the (row, head) unit in blockIdx.x.
-  const int qt = (int)gridDim.y - 1 - (int)blockIdx.y;
-  int row, head;
-  jeff_unit_of(a, rows, blockIdx.x, row, head);
-  const int kvh = min((int)a.gdiv.div((uint32_t)head), a.kv_heads - 1);
-  const int q0 = qt * 16, q = q0 + col;
+  const int kvunits = rows * a.kv_heads;
+  const int sub = (int)blockIdx.x / kvunits, kvu = (int)blockIdx.x - sub * kvunits;
+  const int row = (int)a.kvdiv.div((uint32_t)kvu), kvh = kvu - row * a.kv_heads;
+  const int tiles = 4 / hg;  // query tiles per workgroup
+  const int yg = (int)gridDim.y - 1 - (int)blockIdx.y;
+  const int head = kvh * a.groups + sub * hg + wave % hg;
+  const int q0 = 16 * (yg * tiles + wave / hg), q = q0 + col;
   const float *Q = static_cast<const float *>(a.q) + row * a.q_row + (size_t)head * hd * L;
   const float *Gt = static_cast<const float *>(a.gate) + row * a.q_row + (size_t)head * hd * L;
-  const float *V = static_cast<const float *>(a.v) + row * a.kv_row + (size_t)kvh * a.kv_head;
-  const int Lp = (L + 15) & ~15;
-  const float *KP = kp + ((size_t)row * a.kv_heads + kvh) * (size_t)Lp * HDP;
-  const uint32_t *rbits = kbits + (size_t)row * ((L + 31) / 32);
   float *OUT = a.out + row * a.q_row + (size_t)head * hd * L;
-  float *ww = smem + wave * (2 * QS * 64);  // this wave's rows: its K and V slices
+  const int nt = (L + 31) / 32;
+  const unsigned char *unit = planes + (size_t)kvu * nt * kJeffTileBytes;
+  const int *uexp = vexp + (size_t)kvu * nt;
+  const uint32_t *rbits = kbits + (size_t)row * nt;
 
-  // This lane's features in both products: step (c, e) of the 16x16x4 MFMA
-  // chain uses feature d0 + 16c + e (the prep workspace's run order).
-  const int d0 = wave * DS + 4 * grp;
-  // Along-token tasks of the wave's slice (Q, gate, output): task t is
-  // feature wave*DS + (lane >> 2) + 16t, tokens q0 + 4*(lane & 3) .. + 3.
-  const int tdl = lane >> 2, tg4 = lane & 3;
-
-  // -------- loads that need nothing: the row's key span, the diagonal key
-  // tile (the walk runs from it down to the row's first active key).
-  // K: key k0 + col, features d0 + 16c .. + 3 = run c of the tile's block
-  // for this wave, chunk lane (zero past hd and past L). V: V[wave*DS + 16j
-  // + col][k0 + 4*grp .. + 3].
-  const __amdgpu_buffer_rsrc_t rk = buffer_rsrc(KP, (uint32_t)((size_t)Lp * HDP * 4));
-  const __amdgpu_buffer_rsrc_t rv = buffer_rsrc(V, (uint32_t)((size_t)hd * L * 4));
-  const int okk = wave * 4096 + lane * 16;
-  const int ovv = ((wave * DS + col) * L + 4 * grp) * 4;
-  f32x4 kc[QS / 4], vc[NB];
-  auto fetch = [&](int k0, f32x4 (&kr)[QS / 4], f32x4 (&vr)[NB]) {
-    k0 = __builtin_amdgcn_readfirstlane(k0);  // uniform: scalar offsets, no waterfall
-#pragma unroll
-    for (int c = 0; c < QS / 4; ++c) kr[c] = buffer_load4(rk, okk + 1024 * c, k0 * HDP * 4);
-#pragma unroll
-    for (int j = 0; j < NB; ++j) vr[j] = buffer_load4(rv, ovv + j * 16 * L * 4, k0 * 4);
-  };
-  // The Q tile's HBM round trip starts with the item (wasted only for a
-  // tile with no key, which never reads it).
+  // The Q tile and its norm weights: issued first (wasted only for a tile
+  // with no key). Task e = lane + 64 u: feature e / 4, queries q0 + 4 (e % 4) ..
+  // + 3, features past hd read 0; weights of features 32 s + 8 grp .. + 7.
   const __amdgpu_buffer_rsrc_t rq = buffer_rsrc(Q, (uint32_t)((size_t)hd * L * 4));
-  const int otask = ((wave * DS + tdl) * L + 4 * tg4) * 4;  // byte offset of task 0
-  f32x4 qx[NB];
+  const __amdgpu_buffer_rsrc_t rn = buffer_rsrc(a.q_norm, (uint32_t)(hd * 4));
+  f32x4 qx[HDP / 16], wv[HDP / 16];
 #pragma unroll
-  for (int t = 0; t < NB; ++t) qx[t] = buffer_load4(rq, otask + t * 16 * L * 4, q0 * 4);
+  for (int u = 0; u < HDP / 16; ++u)
+    qx[u] = buffer_load4(rq, ((lane >> 2) * L + 4 * (lane & 3)) * 4, u * 16 * L * 4 + q0 * 4);
+#pragma unroll
+  for (int c = 0; c < HDP / 16; ++c)
+    wv[c] = buffer_load4(rn, (8 * grp + 4 * (c & 1)) * 4, 128 * (c / 2));
+
   const int first = spans[2 * row], last = spans[2 * row + 1];
-  fetch(qt * KT, kc, vc);
   const int start = (a.trim && last >= 0) ? first : 0;
   const bool q_live = q < L && q >= start;
-  const int q_last = min(q0 + 15, L - 1);
-  int kt_begin = 0, kt_end = 0;
+  // The workgroup's 32-key tiles: first active key .. last query.
+  int t_begin = 0, t_end = 0;
   {
-    const int kl = min(last, q_last);
-    if (last >= 0 && first <= kl && q_last >= start) {
-      kt_begin = first / KT;
-      kt_end = kl / KT + 1;
+    const int q_hi = min(16 * (yg + 1) * tiles - 1, L - 1), kl = min(last, q_hi);
+    if (last >= 0 && first <= kl && q_hi >= start) {
+      t_begin = first / 32;
+      t_end = kl / 32 + 1;
     }
   }
-  kt_begin = __builtin_amdgcn_readfirstlane(kt_begin);
-  kt_end = __builtin_amdgcn_readfirstlane(kt_end);
-
-  const __amdgpu_buffer_rsrc_t rg = buffer_rsrc(Gt, (uint32_t)((size_t)hd * L * 4));
-  const __amdgpu_buffer_rsrc_t ro = buffer_rsrc(OUT, (uint32_t)((size_t)hd * L * 4));
-  f32x4 gv[NB];
-  auto load_gate = [&]() {
-#pragma unroll
-    for (int t = 0; t < NB; ++t) gv[t] = buffer_load4(rg, otask + t * 16 * L * 4, q0 * 4);
-  };
-  // o * sigmoid(gate) (lib.rs:755-758) for task t, o = O^T * inv; 0 for a
-  // dropped query (q < start). L % 4 == 0: a task's 4 tokens are all in or
-  // all out.
-  auto store_task = [&](int t, f32x4 o) {
-    const int qa = q0 + 4 * tg4, d = wave * DS + tdl + 16 * t;
-    f32x4 r;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r[i] = qa + i < start ? 0.0f : o[i] * fast_sigmoid(gv[t][i]);
-    if (qa < L && d < hd) buffer_store4_nt(r, ro, otask + t * 16 * L * 4, q0 * 4);
-  };
-  if (kt_begin >= kt_end) {
-    // No key at or before these queries: o = 0 (lib.rs:739-743), and
-    // 0 * sigmoid(gate) is 0 for every gate but NaN (sigmoid is in [0, 1],
-    // also at +-inf), which it propagates: no exponential needed.
-    load_gate();
-#pragma unroll
-    for (int t = 0; t < NB; ++t) {
-      const int qa = q0 + 4 * tg4, d = wave * DS + tdl + 16 * t;
-      f32x4 r;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) r[i] = (qa + i >= start && gv[t][i] != gv[t][i]) ? gv[t][i] : 0.0f;
-      if (qa < L && d < hd) buffer_store4_nt(r, ro, otask + t * 16 * L * 4, q0 * 4);
-    }
-    return;
-  }
-
-  // -------- Q: the wave's slice along tokens, transposed through its LDS
-  // rows into this lane's B operands (feature d0 + 16c + e of query q0 +
-  // col; features past hd read as 0); its norm weights and, where the RoPE
-  // partners sit in the same lane (rot/2 = 16 or 32: partner of step (c, e)
-  // is (c + rot/32, e)), its table entries.
-  const int rh = a.rot_half;
-  const bool rope = a.cos_t != nullptr && rh > 0;
-  const bool lane_rope = rh == 16 || rh == 32;
-  const __amdgpu_buffer_rsrc_t rn = buffer_rsrc(a.q_norm, (uint32_t)(hd * 4));
-  f32x4 wv[QS / 4];
-#pragma unroll
-  for (int c = 0; c < QS / 4; ++c) wv[c] = buffer_load4(rn, (d0 + 16 * c) * 4, 0);
-  f32x4 tc[2], ts[2];  // wave 0, lane_rope: table entries of pairs i = 4*grp + 16c + e, c < rh/16
-  if (rope && lane_rope && wave == 0) {
-    const size_t pos = (size_t)min(max(q - start, 0), L - 1) * rh;
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int i = min(4 * grp + 16 * c, rh - 4);
-      tc[c] = *reinterpret_cast<const f32x4 *>(a.cos_t + pos + i);
-      ts[c] = *reinterpret_cast<const f32x4 *>(a.sin_t + pos + i);
-    }
-  }
-#pragma unroll
-  for (int t = 0; t < NB; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ww[(4 * tg4 + i) * QW + tdl + 16 * t] = qx[t][i];
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  float qv[QS];
-#pragma unroll
-  for (int c = 0; c < QS / 4; ++c) {
-    const f32x4 y = *reinterpret_cast<const f32x4 *>(ww + col * QW + 4 * grp + 16 * c);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) qv[4 * c + e] = y[e];
-  }
-
-  // -------- RMSNorm (lib.rs:676-691): the sum of squares over the four
-  // waves' slices through LDS, then partial RoPE (692-709).
-  float ss = 0.0f;
-#pragma unroll
-  for (int c = 0; c < QS / 4; ++c)
-    ss += qv[4 * c] * qv[4 * c] + qv[4 * c + 1] * qv[4 * c + 1] + qv[4 * c + 2] * qv[4 * c + 2] +
-          qv[4 * c + 3] * qv[4 * c + 3];
-  ss = pair_sum(pair16_sum(ss));
-  if (grp == 0) s_ssq[wave * 16 + col] = ss;
-  __syncthreads();
-  const float tot = s_ssq[col] + s_ssq[16 + col] + s_ssq[32 + col] + s_ssq[48 + col];
-  const float scale = rms_scale(tot, hd, a.eps);
-  float qreg[QS];
-#pragma unroll
-  for (int c = 0; c < QS / 4; ++c)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int d = d0 + 16 * c + e;
-      qreg[4 * c + e] = (q_live && d < hd) ? rms_apply(qv[4 * c + e], scale, wv[c][e]) : 0.0f;
-    }
-  if (rope && lane_rope) {
-    if (wave == 0 && q_live) {
-      // pc: register-block offset of the partner, a constant in each branch
-      // (a run-time one indexes the register array indirectly).
-      auto rotate = [&](auto pcv) {
-        constexpr int pc = decltype(pcv)::value;
-#pragma unroll
-        for (int c = 0; c < pc; ++c)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float x = qreg[4 * c + e], y = qreg[4 * (c + pc) + e];
-            qreg[4 * c + e] = rope_lo(x, y, tc[c][e], ts[c][e]);
-            qreg[4 * (c + pc) + e] = rope_hi(x, y, tc[c][e], ts[c][e]);
-          }
-      };
-      if (rh == 16)
-        rotate(std::integral_constant<int, 1>{});
-      else
-        rotate(std::integral_constant<int, 2>{});
-    }
-  } else if (rope) {
-    // Any other rotary width: rotate the normalized rows of the whole tile
-    // in LDS (the wave rows are free again).
-    float *Qs = smem;
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < QS / 4; ++c)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) Qs[col * QP + d0 + 16 * c + e] = qreg[4 * c + e];
-    __syncthreads();
-    const int qi = tid & 15, qa = q0 + qi;
-    if (qa < L && qa >= start) {
-      const size_t pq = (size_t)(qa - start) * rh;
-      float *qr = Qs + qi * QP;
-      for (int i = tid >> 4; i < rh; i += 16) {
-        const float x = qr[i], y = qr[i + rh];
-        const float c = a.cos_t[pq + i], sn = a.sin_t[pq + i];
-        qr[i] = rope_lo(x, y, c, sn);
-        qr[i + rh] = rope_hi(x, y, c, sn);
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < QS / 4; ++c)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) qreg[4 * c + e] = Qs[col * QP + d0 + 16 * c + e];
-    __syncthreads();  // the tile rows become wave rows again
-  }
-  f32x4 *sx = reinterpret_cast<f32x4 *>(smem + KVAREA);
-
-  // The next key tile's K and V go into this wave's LDS slices with LDS-DMA
-  // loads (no registers held; the wave reads back exactly the bytes it
-  // loaded, so it only waits for its own loads). Issued once the previous
-  // contents are in registers, one tile ahead of their use.
-  unsigned char *const kv_lds = reinterpret_cast<unsigned char *>(smem) + wave * KVW * 4;
-  const u32x4r rkw = rsrc_words(KP, (uint32_t)((size_t)Lp * HDP * 4));
-  const u32x4r rvw = rsrc_words(V, (uint32_t)((size_t)hd * L * 4));
-  auto prefetch = [&](int k0) {
-    k0 = __builtin_amdgcn_readfirstlane(k0);
-    // One offset register per lane (okk, ovv); the per-load steps go in the
-    // scalar offset.
-#pragma unroll
-    for (int c = 0; c < QS / 4; ++c)
-      load_lds16(rkw, (uint32_t)okk, (uint32_t)(k0 * HDP * 4 + 1024 * c), kv_lds + 1024 * c);
-#pragma unroll
-    for (int j = 0; j < NB; ++j)
-      load_lds16(rvw, (uint32_t)ovv, (uint32_t)(k0 * 4 + j * 16 * L * 4),
-                 kv_lds + QS * 256 + 1024 * j);
-  };
-  auto take = [&]() {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-    for (int c = 0; c < QS / 4; ++c)
-      kc[c] = *reinterpret_cast<const f32x4 *>(kv_lds + 1024 * c + 16 * lane);
-#pragma unroll
-    for (int j = 0; j < NB; ++j)
-      vc[j] = *reinterpret_cast<const f32x4 *>(kv_lds + QS * 256 + 1024 * j + 16 * lane);
-  };
-  // The gate tasks of the wave's slice go into its V slice during the last
-  // step (read back after the walk).
-  const u32x4r rgw = rsrc_words(Gt, (uint32_t)((size_t)hd * L * 4));
-  auto gate_to_lds = [&]() {
-#pragma unroll
-    for (int t = 0; t < NB; ++t)
-      load_lds16(rgw, (uint32_t)otask, (uint32_t)(q0 * 4 + t * 16 * L * 4),
-                 kv_lds + QS * 256 + 1024 * t);
-  };
-
-  // Keep word of a 16-key tile for query col: active key (the prep's bits:
-  // mask != 0, zero past L), key <= query (lib.rs:716). Keys before `start`
-  // are inactive by definition of start. The bits word is loaded one tile
-  // ahead (bits_of) and turned into the word after that tile's products.
-  auto bits_of = [&](int kt) -> uint32_t { return rbits[kt >> 1]; };
-  auto keep_word = [&](int kt, uint32_t word) -> uint32_t {
-    const uint32_t abits = (word >> (16 * (kt & 1))) & 0xffffu;
-    return q_live ? (abits & range_bits(0, q - kt * KT)) : 0u;
-  };
+  t_begin = __builtin_amdgcn_readfirstlane(t_begin);
+  t_end = __builtin_amdgcn_readfirstlane(t_end);
 
   f32x4 O[NB];
 #pragma unroll
   for (int j = 0; j < NB; ++j) O[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   float m = kNoMax, l = 0.0f;  // l: this lane's share of the row sum
-  const float c1 = a.c1;
-
-  // -------- the walk, from the last key tile down (exponents against a
-  // lazily moved reference, as in the Laya kernel; the order of the keys
-  // only moves rounding). A workgroup whose kept scores sum to NaN or inf
-  // stops computing; it, or one whose O took a NaN or inf, redoes the tile
-  // with the reference's exact semantics afterwards. The gate loads go out
-  // with the last tile. The first tile is in registers (loaded with the
-  // item); every later one comes through LDS, prefetched a step ahead (the
-  // prologue's last use of the wave rows was before its barrier).
-  const int kt_hi = kt_end - 1;
-  if (kt_hi != qt) fetch(kt_hi * KT, kc, vc);  // the span ends before the diagonal
-  if (kt_hi > kt_begin) prefetch((kt_hi - 1) * KT);
-  uint32_t w = keep_word(kt_hi, bits_of(kt_hi));
-  bool tainted = false;  // workgroup-uniform
-  int xb = 0;            // exchange buffer
-  // One step per key tile. The first is peeled off (FIRST): its K and V come
-  // from registers, every later one from the slices. So no vector-memory
-  // load that the compiler tracks is in flight inside the loop, and the
-  // waits it inserts there never hold up the next tile's LDS-DMA loads.
-  auto step = [&](int kt, auto first) {
-    constexpr bool FIRST = decltype(first)::value;
-    const bool more = kt > kt_begin;
-    uint32_t bnext = 0u;
-    if constexpr (!FIRST) {
-      take();
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slices are in registers
-    }
-    if (more) {
-      if constexpr (!FIRST) prefetch((kt - 1) * KT);
-      bnext = bits_of(kt - 1);
-    } else {
-      gate_to_lds();
-    }
-    if (kt * KT + KT > L) {  // the row's last, partial tile: V past L is another feature's
+  bool tainted = false;        // wave-uniform
+  if (t_begin < t_end) {
+    f16x8 qh[ST], ql[ST];
+    const int eq = spans[-2], en = eq + spans[-1];
+    const float c1 = ldexpf(a.c1, en - 2 * kJeffNormUp);
+    {
+      // RMSNorm (lib.rs:676-691) and partial RoPE (692-709): the queries
+      // transposed through the wave's LDS rows into the B operands' order,
+      // lane (col, grp) holding features 32 s + 8 grp .. + 7 of query col.
+      constexpr int QP = HDP + 4;
+      const int rh = a.rot_half;
+      const bool rope = a.cos_t != nullptr && rh > 0;
+      const size_t pos = (size_t)min(max(q - start, 0), L - 1) * rh;
+      f32x4 tc[2], ts[2];
+      if (rope && rh == 32) {
 #pragma unroll
-      for (int j = 0; j < NB; ++j)
+        for (int h = 0; h < 2; ++h) {
+          tc[h] = *reinterpret_cast<const f32x4 *>(a.cos_t + pos + 8 * grp + 4 * h);
+          ts[h] = *reinterpret_cast<const f32x4 *>(a.sin_t + pos + 8 * grp + 4 * h);
+        }
+      }
+      auto settle = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      };
 #pragma unroll
-        for (int t = 0; t < 4; ++t) vc[j][t] = kt * KT + 4 * grp + t < L ? vc[j][t] : 0.0f;
-    }
-    if (!tainted && __ballot(w != 0u) != 0) {  // workgroup-uniform: every wave has the same w
-      f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = {0.0f, 0.0f, 0.0f, 0.0f};
+      for (int u = 0; u < HDP / 16; ++u)
 #pragma unroll
-      for (int c = 0; c < QS / 4; ++c) {
+        for (int i = 0; i < 4; ++i)
+          ws[(4 * (lane & 3) + i) * QP + (lane >> 2) + 16 * u] = qx[u][i];
+      settle();
+      float *const qr = ws + col * QP;
+      float ss = 0.0f;
+#pragma unroll
+      for (int c = 0; c < 2 * ST; ++c) {
+        qx[c] = *reinterpret_cast<const f32x4 *>(qr + 32 * (c / 2) + 8 * grp + 4 * (c & 1));
+        ss += qx[c][0] * qx[c][0] + qx[c][1] * qx[c][1] + qx[c][2] * qx[c][2] + qx[c][3] * qx[c][3];
+      }
+      const float scale = rms_scale(pair_sum(pair16_sum(ss)), hd, a.eps);
+#pragma unroll
+      for (int c = 0; c < 2 * ST; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          qx[c][e] = q_live && 32 * (c / 2) + 8 * grp + 4 * (c & 1) + e < hd
+                         ? rms_apply(qx[c][e], scale, wv[c][e])
+                         : 0.0f;
+      if (rope && rh == 32) {
+        if (q_live) {  // pairs (i, i + 32): the same element of steps 0 and 1
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float x = qx[h][e], y = qx[2 + h][e];
+              qx[h][e] = rope_lo(x, y, tc[h][e], ts[h][e]);
+              qx[2 + h][e] = rope_hi(x, y, tc[h][e], ts[h][e]);
+            }
+        }
+      } else if (rope) {
+#pragma unroll
+        for (int c = 0; c < 2 * ST; ++c)
+          *reinterpret_cast<f32x4 *>(qr + 32 * (c / 2) + 8 * grp + 4 * (c & 1)) = qx[c];
+        settle();
+        if (q_live)
+          for (int i = grp; i < rh; i += 4) {
+            const float x = qr[i], y = qr[i + rh], cc = a.cos_t[pos + i], sn = a.sin_t[pos + i];
+            qr[i] = rope_lo(x, y, cc, sn);
+            qr[i + rh] = rope_hi(x, y, cc, sn);
+          }
+        settle();
+#pragma unroll
+        for (int c = 0; c < 2 * ST; ++c)
+          qx[c] = *reinterpret_cast<const f32x4 *>(qr + 32 * (c / 2) + 8 * grp + 4 * (c & 1));
+      }
+      const float sc = pow2i(kJeffNormUp - eq);
+#pragma unroll
+      for (int c = 0; c < 2 * ST; ++c) {
+        f16x4 h, lo;
+        split_f16(qx[c], sc, h, lo);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          if (c & 1)
-            s1 = mfma_16x16x4(kc[c][e], qreg[4 * c + e], s1);
-          else
-            s0 = mfma_16x16x4(kc[c][e], qreg[4 * c + e], s0);
+          qh[c / 2][4 * (c & 1) + e] = h[e];
+          ql[c / 2][4 * (c & 1) + e] = lo[e];
         }
-      }
-      sx[(xb * 4 + wave) * 64 + lane] = s0 + s1;
-      __syncthreads();
-      f32x4 s = sx[(xb * 4 + 0) * 64 + lane];
-#pragma unroll
-      for (int v = 1; v < 4; ++v) s += sx[(xb * 4 + v) * 64 + lane];
-      xb ^= 1;
-      // lane group g holds keys 4g + r of its query
-      if (__ballot(q_live && w != 0xffffu) != 0) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[r] = ((w >> (4 * grp + r)) & 1u) ? s[r] : -INFINITY;
-      }
-      f32x4 ex;
-      float rs = 0.0f;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        ex[r] = fast_exp2(__builtin_fmaf(s[r], c1, -m));
-        rs += ex[r];
-      }
-      bool ok = true;
-      if (__ballot(q_live && !(rs <= kLazyLimit)) != 0) {
-        const float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-        const float mxs = pair_max(pair16_max(mx)) * c1;
-        const bool need = mxs > m + kRescaleSlack;
-        const float mn = need ? mxs : m;
-        rs = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          ex[r] = fast_exp2(__builtin_fmaf(s[r], c1, -mn));
-          rs += ex[r];
-        }
-        if (__ballot(q_live && !__builtin_isfinite(rs)) != 0) {
-          tainted = true;
-          ok = false;
-        } else {
-          const float alpha = fast_exp2(m - mn);  // exactly 1 where the reference stays
-#pragma unroll
-          for (int j = 0; j < NB; ++j) O[j] *= alpha;
-          l *= alpha;
-          m = mn;
-        }
-      }
-      if (ok) {
-        l += rs;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int j = 0; j < NB; ++j) O[j] = mfma_16x16x4(vc[j][r], ex[r], O[j]);
       }
     }
-    if (more) w = keep_word(kt - 1, bnext);
-  };
-  __builtin_amdgcn_s_setprio(0);
-  step(kt_hi, std::true_type{});
-  for (int kt = kt_hi - 1; kt >= kt_begin; --kt) step(kt, std::false_type{});
-  __builtin_amdgcn_s_setprio(3);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the gate slice, and no LDS-DMA left in flight
+    __syncthreads();  // the wave rows become the tile buffers
 
-  // -------- careful redo (rare): the scores (shared) or this wave's O went
-  // non-finite; one wave redoes the whole tile from global memory.
+    // This wave's share of a half tile's 32 pieces of 1 KB (half 0: K, 1: V).
+    auto load_half = [&](int t, int half) {
+      const u32x4r r = rsrc_words(unit + (size_t)t * kJeffTileBytes + half * kJeffTileV, kJeffTileV);
+      unsigned char *dst = lds + half * kJeffTileV;
+#pragma unroll
+      for (int i = 0; i < PW; ++i)
+        load_lds16(r, 16u * lane, (uint32_t)(1024 * (PW * wave + i)), dst + 1024 * (PW * wave + i));
+    };
+    // This wave's loads have landed (but for its youngest half tile's when
+    // `young`) and its LDS reads are done, and so for every wave.
+    auto arrive = [&](bool young) {
+      if (young)
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PW) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    };
+    load_half(t_begin, 0);
+    load_half(t_begin, 1);
+    int EV = -126;  // O's unit is 2^EV
+    constexpr float kShift = 7.0f, kLimit = 32768.0f;  // probabilities 2^7 up, below fp16's 2^15
+    const unsigned char *const kl = lds + 16 * lane, *const vl = kl + kJeffTileV;
+    uint32_t word_next = rbits[t_begin];  // scalar loads, one tile ahead of their use
+    int ev_next = uexp[t_begin];
+    for (int t = t_begin; t < t_end; ++t) {
+      arrive(t == t_begin);  // K of t; V of t - 1 has been read by every wave
+      if (t > t_begin) load_half(t, 1);
+      const uint32_t word = word_next;
+      const int ev = ev_next;
+      word_next = rbits[min(t + 1, nt - 1)];
+      ev_next = uexp[min(t + 1, nt - 1)];
+      const uint32_t w = q_live ? (word & range_bits(0, q - 32 * t)) : 0u;
+      const bool mine = !tainted && __ballot(w != 0u) != 0;
+      f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = s0;
+      if (mine) {
+        // Three accumulators (even steps, odd steps, cross products): fewer
+        // roundings of the whole sum than one.
+        f32x4 r0 = s0, r1 = s0, u0 = s0, u1 = s0;
+        // Operands two steps ahead of their products (an LDS read takes about
+        // as long as two steps' products when all waves read), and no product
+        // right behind one into the same accumulator (it would wait for that
+        // one's eight passes).
+        f16x8 kx[3][4];
+        auto take = [&](int x) {
+          kx[x % 3][0] = *reinterpret_cast<const f16x8 *>(kl + 2048 * x);
+          kx[x % 3][1] = *reinterpret_cast<const f16x8 *>(kl + 2048 * (ST + x));
+          kx[x % 3][2] = *reinterpret_cast<const f16x8 *>(kl + 2048 * x + 1024);
+          kx[x % 3][3] = *reinterpret_cast<const f16x8 *>(kl + 2048 * (ST + x) + 1024);
+        };
+        take(0);
+        take(1);
+#pragma unroll
+        for (int x = 0; x < ST; ++x) {
+          if (x + 2 < ST) take(x + 2);
+          const f16x8 k0h = kx[x % 3][0], k1h = kx[x % 3][1], k0l = kx[x % 3][2], k1l = kx[x % 3][3];
+          r0 = mfma_16x16x32_f16(k0l, ql[x], r0);
+          r1 = mfma_16x16x32_f16(k1l, ql[x], r1);
+          if (x & 1) {
+            u0 = mfma_16x16x32_f16(k0h, qh[x], u0);
+            u1 = mfma_16x16x32_f16(k1h, qh[x], u1);
+          } else {
+            s0 = mfma_16x16x32_f16(k0h, qh[x], s0);
+            s1 = mfma_16x16x32_f16(k1h, qh[x], s1);
+          }
+          r0 = mfma_16x16x32_f16(k0h, ql[x], r0);
+          r1 = mfma_16x16x32_f16(k1h, ql[x], r1);
+          r0 = mfma_16x16x32_f16(k0l, qh[x], r0);
+          r1 = mfma_16x16x32_f16(k1l, qh[x], r1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        s0 += u0 + r0;
+        s1 += u1 + r1;
+      }
+      arrive(false);  // V of t; K of t has been read by every wave
+      if (t + 1 < t_end) load_half(t + 1, 0);
+      if (mine) {
+        if (__ballot(q_live && w != 0xffffffffu) != 0) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            s0[r] = ((w >> (4 * grp + r)) & 1u) ? s0[r] : -INFINITY;
+            s1[r] = ((w >> (16 + 4 * grp + r)) & 1u) ? s1[r] : -INFINITY;
+          }
+        }
+        f32x4 e0, e1;
+        float rs = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          e0[r] = fast_exp2(__builtin_fmaf(s0[r], c1, -m));
+          e1[r] = fast_exp2(__builtin_fmaf(s1[r], c1, -m));
+          rs += e0[r] + e1[r];
+        }
+        bool ok = true;
+        if (__ballot(q_live && !(rs <= kLimit)) != 0) {
+          // Move the reference where the tile max exceeds it by more than the slack.
+          const float mx = fmaxf(fmaxf(fmaxf(s0[0], s0[1]), fmaxf(s0[2], s0[3])),
+                                 fmaxf(fmaxf(s1[0], s1[1]), fmaxf(s1[2], s1[3])));
+          const float mxs = pair_max(pair16_max(mx)) * c1;
+          const bool need = mxs > m + (kRescaleSlack + kShift);
+          const float mn = need ? mxs - kShift : m;
+          rs = 0.0f;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            e0[r] = fast_exp2(__builtin_fmaf(s0[r], c1, -mn));
+            e1[r] = fast_exp2(__builtin_fmaf(s1[r], c1, -mn));
+            rs += e0[r] + e1[r];
+          }
+          if (__ballot(q_live && !__builtin_isfinite(rs)) != 0) {
+            tainted = true;
+            ok = false;
+          } else {
+            const float alpha = fast_exp2(m - mn);  // exactly 1 where the reference stays
+#pragma unroll
+            for (int j = 0; j < NB; ++j) O[j] *= alpha;
+            l *= alpha;
+            m = mn;
+          }
+        }
+        if (ok) {
+          l += rs;
+          if (ev > EV) {  // a larger unit for O; a smaller tile's goes into its probabilities
+            const float f = ldexpf(1.0f, EV - ev);
+#pragma unroll
+            for (int j = 0; j < NB; ++j) O[j] *= f;
+            EV = ev;
+          }
+          const float f = ldexpf(1.0f, ev - EV);
+          f16x4 h0, l0, h1, l1;
+          split_f16(e0, f, h0, l0);
+          split_f16(e1, f, h1, l1);
+          const f16x8 ph = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+          const f16x8 pl = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+          f16x8 vx[2][8];
+          auto take = [&](int g) {  // the hi and lo blocks of features 64 g ..
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+              vx[g & 1][i] = *reinterpret_cast<const f16x8 *>(vl + 2048 * (4 * g + (i & 3)) + 1024 * (i >> 2));
+          };
+          take(0);
+#pragma unroll
+          for (int g = 0; g < NB / 4; ++g) {
+            if (g + 1 < NB / 4) take(g + 1);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) O[4 * g + i] = mfma_16x16x32_f16(vx[g & 1][i], pl, O[4 * g + i]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) O[4 * g + i] = mfma_16x16x32_f16(vx[g & 1][4 + i], ph, O[4 * g + i]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) O[4 * g + i] = mfma_16x16x32_f16(vx[g & 1][i], ph, O[4 * g + i]);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+      }
+    }
+    __syncthreads();  // the tile buffers become wave rows again
+    const float f = pow2i(EV);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) O[j] *= f;
+  }
+  if (q0 >= L) return;  // no barrier follows
+
+  // -------- careful redo (rare), out of line: NaN / inf among this wave's
+  // kept scores or values.
   bool bad = false;
 #pragma unroll
   for (int j = 0; j < NB; ++j)
 #pragma unroll
     for (int r = 0; r < 4; ++r) bad |= !__builtin_isfinite(O[j][r]);
-  // Flags and the row sums' inverses go into the exchange buffer that the
-  // last exchange did not use: every wave finished reading it before that
-  // exchange's barrier.
-  float *const xs = smem + KVAREA + xb * (SX / 2);
-  int *const s_flag = reinterpret_cast<int *>(xs);
-  const bool wbad = __ballot(q_live && bad) != 0;
-  if (lane == 0) s_flag[wave] = wbad ? 1 : 0;
-  __syncthreads();
-  if (tainted || (s_flag[0] | s_flag[1] | s_flag[2] | s_flag[3]) != 0) {
-    if (wave == 0) jeff_redo_wave<HDP, true, 1>(kernel_jeff_args(), kp, row, head, q0, kt_begin, kt_end, start, smem);
+  if (tainted || __ballot(q_live && bad) != 0) {
+    jeff_redo_wave<HDP, true, 1>(kernel_jeff_args(), nullptr, row, head, q0, 2 * t_begin, 2 * t_end,
+                                 start, ws);
     return;
   }
-
-  // -------- o / sum (0 when nothing was kept), sigmoid gate, store: O^T
-  // through the wave's rows [feature][query] so that each task stores 4
-  // tokens of one feature.
-  float *const s_inv = xs + 64;
+  // -------- o / sum (0 when nothing was kept), sigmoid gate, store
   const float lt = pair_sum(pair16_sum(l));
-  if (grp == 0) s_inv[wave * 16 + col] = lt > 0.0f ? fast_rcp(lt) : 0.0f;
-#pragma unroll
-  for (int j = 0; j < NB; ++j)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) ww[(16 * j + 4 * grp + r) * OW + col] = O[j][r];
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const f32x4 inv4 = *reinterpret_cast<const f32x4 *>(s_inv + wave * 16 + 4 * tg4);
-#pragma unroll
-  for (int t = 0; t < NB; ++t)
-    gv[t] = *reinterpret_cast<const f32x4 *>(kv_lds + QS * 256 + 1024 * t + 16 * lane);
-#pragma unroll
-  for (int t = 0; t < NB; ++t) {
-    const f32x4 o = *reinterpret_cast<const f32x4 *>(ww + (tdl + 16 * t) * OW + 4 * tg4);
-    store_task(t, o * inv4);
-  }
+  const float inv = lt > 0.0f ? fast_rcp(lt) : 0.0f;
+  jeff_store<HDP, true>(a, Gt, OUT, q0, start, ws, O, inv);
 }
 
 // ------------------------------------------- f32 attention, fused, hd 256
@@ -2844,7 +2763,7 @@ __global__ __launch_bounds__(256, 2) void jeff_bf16_exact_kernel(const JeffArgs 
 // ----------------------------------------------------------------- launchers
 
 // Workspace: the prepared keys (per row and kv head, keys rounded up to 16
-// for the split-head kernel's padded blocks), then one (first, last) key
+// for whole 16-key blocks), then one (first, last) key
 // span per row and the rows' active-key bits (32 keys per word).
 static size_t jeff_kp_main_bytes(const JeffArgs &a, int rows, int hd_pad, bool bf16) {
   const size_t Lp = ((size_t)a.L + 15) & ~(size_t)15;
@@ -2872,10 +2791,9 @@ static hipError_t launch_jeff_f32_hd(const JeffArgs &a, int rows, float *kp, hip
   if constexpr (HDP == 256) {
     // Grids of at most two workgroups per CU (one row of C4 is 128) take
     // the fused kernel: one launch, no K prep, every query tile's key range
-    // on eight wavefronts. Larger grids keep the K prep and the split-head
-    // kernel, which holds four workgroups per CU (the fused kernel's 256
-    // registers per wave allow two) and reads each prepared key tile with
-    // 1 KB loads instead of normalizing it again for every query tile.
+    // on eight wavefronts. Larger grids take the prep and the split
+    // kernel, whose tiles are normalized and split once instead of for
+    // every query tile.
     const int rb = a.cos_t == nullptr ? 0 : (a.rot_half % 16 == 0 ? a.rot_half / 16 : -1);
     const long items = (long)nq * rows * a.heads;
     const bool div_ok = (uint64_t)rows * a.heads * a.heads <= ((uint64_t)1 << 32);
@@ -2907,20 +2825,25 @@ static hipError_t launch_jeff_f32_hd(const JeffArgs &a, int rows, float *kp, hip
                               ev.start, ev.stop, 0, a, rows);
       return hipGetLastError();
     }
-    // Buffer offsets of the split kernel: one head's (hd, L) block and one
-    // kv head's padded K blocks within 2 GiB (checked above, L + 15 < 2^21).
-    if (vec && div_ok) {
-      int *spans = reinterpret_cast<int *>(reinterpret_cast<char *>(kp) +
-                                           jeff_kp_main_bytes(a, rows, HDP, false));
+    // The split kernel takes every length and alignment (its 16-byte accesses
+    // along tokens need dword alignment only); buffer offsets need one head's
+    // (hd, L) block within 2 GiB.
+    if (((size_t)a.L + 15) * (size_t)HDP * 4 < ((size_t)1 << 31) && div_ok &&
+        a.kv_heads <= 32767) {
+      const int nt = (a.L + 31) / 32;
+      const size_t tiles = (size_t)rows * a.kv_heads * nt;
+      unsigned char *planes = reinterpret_cast<unsigned char *>(kp);
+      int *vexp = reinterpret_cast<int *>(planes + tiles * kJeffTileBytes);
+      int *spans = vexp + tiles + 2;
       uint32_t *kbits = reinterpret_cast<uint32_t *>(spans + 2 * rows);
-      const dim3 sp((a.L + 31) / 32, a.kv_heads, rows);
-      hipExtLaunchKernelGGL(jeff_k_prep_split_kernel, sp, dim3(256), 0, stream, ev.start, nullptr,
-                            0, a, kp, spans, kbits);
+      hipExtLaunchKernelGGL(jeff_k_prep_split_kernel, dim3(nt, 2 * a.kv_heads, rows), dim3(256), 0,
+                            stream, ev.start, nullptr, 0, a, planes, vexp, spans, kbits);
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
-      const dim3 sgrid(rows * a.heads, nq);
-      hipExtLaunchKernelGGL((jeff_split_f32_kernel<HDP>), sgrid, dim3(256), 0, stream, nullptr,
-                            ev.stop, 0, a, kp, spans, kbits, rows);
+      const unsigned units = (unsigned)(rows * a.kv_heads * (a.groups / a.heads_per_group));
+      const unsigned n4 = (unsigned)((nq * a.heads_per_group + 3) / 4);
+      hipExtLaunchKernelGGL((jeff_split_f32_kernel<HDP>), dim3(units, n4), dim3(256), 0, stream,
+                            nullptr, ev.stop, 0, a, planes, vexp, spans, kbits, rows);
       return hipGetLastError();
     }
   }
@@ -2960,8 +2883,12 @@ size_t jeff_bf16_flags_offset(const JeffArgs &a, int rows) {
 size_t jeff_kp_bytes(const JeffArgs &a, int rows, int hd_pad, bool bf16) {
   if (bf16 && hd_pad == 256 && jeff_bf16_wide_fits(a))
     return jeff_bf16_flags_offset(a, rows) + jeff_bf16_wide_flag_count(a, rows) * sizeof(int);
-  return jeff_kp_main_bytes(a, rows, hd_pad, bf16) + (size_t)rows * 2 * sizeof(int) +
-         (size_t)rows * ((a.L + 31) / 32) * sizeof(uint32_t);
+  const size_t nt = ((size_t)a.L + 31) / 32;
+  const size_t main = jeff_kp_main_bytes(a, rows, hd_pad, bf16);
+  const size_t tiles = (size_t)rows * a.kv_heads * nt;  // f32 at hd 256: planes and V exponents
+  const size_t split = !bf16 && hd_pad == 256 ? tiles * (kJeffTileBytes + sizeof(int)) + 2 * sizeof(int) : 0;
+  return (main > split ? main : split) + (size_t)rows * 2 * sizeof(int) +
+         (size_t)rows * nt * sizeof(uint32_t);
 }
 
 template <int HDP>
