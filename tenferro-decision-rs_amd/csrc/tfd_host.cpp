@@ -947,6 +947,32 @@ int jeff_layer(tfd_ctx *c, size_t rows, size_t length, size_t hidden, size_t hea
   return finish(c, flags, out, out_d, sizeof(float) * xn);
 }
 
+// Whether a linear takes the few-column kernel: up to 256 columns its single
+// memory round trip beats the f32 GEMM's k loop (2304 x 96 x 768 16 -> 5 us,
+// 2304 x 200 15 -> 9 us; at 400 columns its re-reads of both operands take
+// longer than the GEMM).
+bool skinny_fits(size_t in, size_t out, size_t cols, const float *w, const float *x) {
+  return cols <= 256 && in % 4 == 0 && in > 0 && in <= (size_t)INT32_MAX / 4 &&
+         out <= (size_t)INT32_MAX / 4 && aligned16(w) && aligned16(x);
+}
+
+tfd::SkinnyArgs skinny_args(const float *w, const float *b, size_t in, size_t out, const float *x,
+                            size_t cols, float *y, int act, bool accumulate) {
+  tfd::SkinnyArgs g{};
+  g.w = w;
+  g.x = x;
+  g.k = (int)in;
+  g.m = (int)out;
+  g.n = (int)cols;
+  g.ldx = in;
+  g.out = y;
+  g.ldc = out;
+  g.bias = b;
+  g.act = act;
+  g.accumulate = accumulate ? 1 : 0;
+  return g;
+}
+
 // ------------------------------------------------------------ model forward
 
 // LayerNorm columns (see tfd::NormArgs) on the context's stream.
@@ -975,6 +1001,11 @@ int norm_cols(tfd_ctx *c, const float *x, const int *map, long cols, size_t d, c
 // the forward applies to its result). `accumulate`: y += W^T x instead.
 int linear_cols(tfd_ctx *c, const float *w, const float *b, size_t in, size_t out,
                 const float *x, size_t cols, float *y, int act, bool accumulate = false) {
+  if (skinny_fits(in, out, cols, w, x)) {
+    tfd::SkinnyArgs g = skinny_args(w, b, in, out, x, cols, y, act, accumulate);
+    TFD_HIP(c, tfd::launch_skinny(g, c->cus, c->stream), "skinny launch");
+    return TFD_OK;
+  }
   int rc = gemm(c, true, false, out, cols, in, w, in, 0, x, in, 0, y, out, 0, 1,
                 accumulate ? 1.0f : 0.0f);
   if (rc) return rc;
@@ -1166,6 +1197,50 @@ int laya_forward(tfd_ctx *c, const tfd_laya_model *m, const int64_t *ids, const 
     if (m->n_layers) p_wi.rows += 32;  // each GeGLU half is padded to whole blocks
     if ((rc = reserve_planes(c, {&p_qkv, &p_wo, &p_wi, &p_wm, &p_x, &p_g}))) return rc;
   }
+  // Short batches: LayerNorm, the column moves around attention, GeGLU and
+  // the residual adds inside the few-column linears, four launches and the
+  // attention per layer instead of ten.
+  bool small = Tc <= 256 && d % 4 == 0 && d <= (size_t)tfd::kSkinnyNormMax && I % 4 == 0;
+  for (size_t i = 0; i < m->n_layers; ++i) {
+    const tfd_laya_encoder_layer &l = m->layers[i];
+    for (const float *p : {l.attn_norm_w, l.attn_norm_b, l.wqkv, l.wo, l.mlp_norm_w, l.mlp_norm_b,
+                           l.wi, l.wo_mlp})
+      small = small && aligned16(p);
+  }
+  for (size_t i = 0; i < m->n_head_layers; ++i) {
+    const tfd_laya_head_layer &hl = m->head[i];
+    small = small && hl.ff % 4 == 0;
+    for (const float *p : {hl.norm1_w, hl.norm1_b, hl.in_proj_w, hl.out_proj_w, hl.norm2_w,
+                           hl.norm2_b, hl.linear1_w, hl.linear2_w})
+      small = small && aligned16(p);
+  }
+  // y = f(LN(in) W (+ b)); nw null: no norm. half: GeGLU. map: y's columns.
+  auto norm_linear = [&](const float *in, const float *nw, const float *nb, const float *w,
+                         const float *b, size_t out, float *y, int act, size_t half,
+                         const int *map) {
+    tfd::SkinnyArgs sa = skinny_args(w, b, d, half ? half : out, in, Tc, y, act, false);
+    sa.ln_w = nw;
+    sa.ln_b = nb;
+    sa.eps = eps;
+    sa.half = (int)half;
+    sa.map = map;
+    TFD_HIP(c, tfd::launch_skinny(sa, c->cus, c->stream), "skinny launch");
+    return (int)TFD_OK;
+  };
+  auto small_attention = [&](const float *in, const float *nw, const float *nb, size_t heads,
+                             int64_t window, const float *w_in, const float *b_in,
+                             const float *w_out, const float *b_out, uint32_t rope_bits,
+                             float *res) {
+    int r = norm_linear(in, nw, nb, w_in, b_in, 3 * d, qkv_f, tfd::kActNone, 0, d_cols);
+    if (r) return r;
+    if ((r = laya_run(c, op, qkv_f, nullptr, d_valid, window, d, heads, L, B, rope_bits, att_f,
+                      TFD_DEVICE_PTRS | TFD_ASYNC, d_need)))
+      return r;
+    tfd::SkinnyArgs sa = skinny_args(w_out, b_out, d, d, att_f, Tc, res, tfd::kActNone, true);
+    sa.xmap = d_cols;
+    TFD_HIP(c, tfd::launch_skinny(sa, c->cus, c->stream), "skinny launch");
+    return (int)TFD_OK;
+  };
   auto norm_planes = [&](const float *in, const float *w, const float *b) {
     tfd::NormArgs na{};
     na.x = in;
@@ -1239,6 +1314,16 @@ int laya_forward(tfd_ctx *c, const tfd_laya_model *m, const int64_t *ids, const 
         return rc;
       continue;
     }
+    if (small) {
+      if ((rc = small_attention(x, l.attn_norm_w, l.attn_norm_b, m->heads,
+                                l.sliding ? (int64_t)m->window : -1, l.wqkv, l.bqkv, l.wo, l.bo,
+                                l.rope_base_bits, x)) ||
+          (rc = norm_linear(x, l.mlp_norm_w, l.mlp_norm_b, l.wi, l.bi, 2 * I, g, tfd::kActNone, I,
+                            nullptr)) ||
+          (rc = linear_cols(c, l.wo_mlp, l.bo_mlp, I, d, g, Tc, x, tfd::kActNone, true)))
+        return rc;
+      continue;
+    }
     const float *ain = x;
     if (l.attn_norm_w) {
       if ((rc = norm_cols(c, x, nullptr, (long)Tc, d, l.attn_norm_w, l.attn_norm_b, eps, a)))
@@ -1274,6 +1359,15 @@ int laya_forward(tfd_ctx *c, const tfd_laya_model *m, const int64_t *ids, const 
           (rc = split_linear(c, w1, p_x, u, hl.linear1_b, tfd::kActRelu)) ||
           (rc = split_rows(c, {split_seg(up, u)})) ||
           (rc = split_linear(c, w2, up, h, hl.linear2_b, tfd::kActNone, true)))
+        return rc;
+      continue;
+    }
+    if (small) {
+      if ((rc = small_attention(h, hl.norm1_w, hl.norm1_b, hl.heads, -1, hl.in_proj_w, hl.in_proj_b,
+                                hl.out_proj_w, hl.out_proj_b, 0u, h)) ||
+          (rc = norm_linear(h, hl.norm2_w, hl.norm2_b, hl.linear1_w, hl.linear1_b, hl.ff, u,
+                            tfd::kActRelu, 0, nullptr)) ||
+          (rc = linear_cols(c, hl.linear2_w, hl.linear2_b, hl.ff, d, u, Tc, h, tfd::kActNone, true)))
         return rc;
       continue;
     }

@@ -301,4 +301,27 @@ bool norm_split_fits(int d);
 hipError_t launch_norm_split(const NormArgs &a, unsigned char *dst, int *exps,
                              hipStream_t stream);
 
+// ------------------------------------------------ f32 linears over few columns
+
+// out[m + ldc * (map ? map[n] : n)] (+)= W_m . X_n (+ bias), activation, with
+// W rows of k contiguous elements and X columns xmap ? xmap[n] : n of stride
+// ldx, LayerNorm'ed first when ln_w is given (k <= kSkinnyNormMax). half > 0:
+// GeGLU of weight rows m and half + m. k % 4 == 0; w, x, ln_w, ln_b 16-byte
+// aligned, ldx % 4 == 0.
+constexpr int kSkinnyNormMax = 1024;
+struct SkinnyArgs {
+  const float *w, *x;
+  const int *xmap;
+  const float *ln_w, *ln_b;
+  float eps;
+  int k, m, n, half;
+  size_t ldx;
+  float *out;
+  size_t ldc;
+  const int *map;
+  const float *bias;
+  int act, accumulate;
+};
+hipError_t launch_skinny(const SkinnyArgs &g, int cus, hipStream_t stream);
+
 }  // namespace tfd
