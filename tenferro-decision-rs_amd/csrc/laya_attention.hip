@@ -27,7 +27,7 @@
 // Measured: L 512 B 8 (padded) 42.5 -> 29.7 us, L 2048 B 4 within +-64 51.4 -> 37 us
 // per call; relative error against 64 bits 2.6e-7 -> 2.0e-7 and 3.4e-7 -> 2.6e-7. Per
 // wave and tile about 180 vector instructions (half of them the split of K
-// and V), 712 LDS cycles per workgroup and the MFMAs now bound it about equally.
+// and V), the LDS reads and the MFMAs follow one another and bound it together.
 #include <type_traits>
 
 #include "tfd_device.hpp"

@@ -1,17 +1,19 @@
 // f32 linears over few columns (a short prompt's tokens, markers, one column
 // per prompt): out (+)= W^T x with everything around it in one launch.
 //
-// At 16 .. 256 columns a linear is bound by latency and by reading its weights
+// At up to 160 columns a linear is bound by latency and by reading its weights
 // once (7 MB take 1.5 us), not by the matrix cores, so the kernel does one
 // memory round trip: a workgroup of 8 waves owns 16 weight rows (GeGLU: 16 of
-// each half) x up to 48 columns, its waves take the 16-k chunks in turn, issue
+// each half) x 16 or 32 columns, its waves take the 16-k chunks in turn, issue
 // all their loads at once (16 bytes per lane, operands straight in the f32
 // matrix cores' layout), and the eight partial sums meet once in LDS. LayerNorm
 // of the columns (their elements are in the waves' registers anyway), the
 // gather of the columns, bias, activation, GeGLU, residual add and the scatter
-// of the result are part of it. Measured at 96 columns (768 -> 2304): 5-6 us
-// with the LayerNorm, against 16 us for the f32 GEMM plus 7 us for the
-// LayerNorm and 4 us for the column moves.
+// of the result are part of it. Measured at 96 columns (768 -> 2304): 14.8 us
+// with LayerNorm and scatter, against 16 us for the f32 GEMM plus 7 us for the
+// LayerNorm and 4 us for the column move; 768 -> 768 12.7 us against 11 + 4. What
+// remains is the chain of dependent round trips: arguments, column map,
+// operands, LDS, store.
 #include "tfd_device.hpp"
 #include "tfd_internal.hpp"
 

@@ -714,9 +714,12 @@ int split_rows(tfd_ctx *c, std::initializer_list<tfd::SplitSeg> list) {
 // Whether a linear of `cols` columns (weights out x in) runs as fp16 planes:
 // from the size where splitting both operands on each call (5 us or more) plus the
 // three fp16 products undercut one f32 product, and a size the planes'
-// 32-bit indices hold.
+// 32-bit indices hold. Whole layers, f32 products -> planes: Laya hidden 512 at
+// 1024 columns 61 -> 67 us and at 1400 102 -> 87; 768 at 896 84 -> 79; 1024 at
+// 512 63 -> 74 and at 640 87 -> 82; Jeff hidden 1024 at 512 91 -> 108 and at
+// 640 139 -> 113.
 bool split_pays(size_t out, size_t in, size_t cols) {
-  return in >= 256 && out >= 256 && cols >= 512 && out * cols >= ((size_t)1 << 19) &&
+  return in >= 256 && out >= 256 && cols >= 640 && out * cols >= ((size_t)5 << 17) &&
          in <= 65536 && out <= ((size_t)1 << 26) && cols <= ((size_t)1 << 26);
 }
 
@@ -947,12 +950,18 @@ int jeff_layer(tfd_ctx *c, size_t rows, size_t length, size_t hidden, size_t hea
   return finish(c, flags, out, out_d, sizeof(float) * xn);
 }
 
-// Whether a linear takes the few-column kernel: up to 256 columns its single
-// memory round trip beats the f32 GEMM's k loop (2304 x 96 x 768 16 -> 5 us,
-// 2304 x 200 15 -> 9 us; at 400 columns its re-reads of both operands take
-// longer than the GEMM).
+// Columns up to which the few-column kernels' single memory round trip beats
+// the f32 GEMMs, norms and moves; beyond it their workgroups take several
+// rounds over the chip and re-read both operands. Forwards of 22 layers, GEMMs
+// -> these: hidden 768 at 96 columns 2118 -> 1541 us, 160 2175 -> 2107, 176
+// 2182 -> 2402; hidden 384 at 160 1318 -> 1237, 224 1341 -> 1385; hidden 1024
+// (LayerNorm over twice the registers) at 96 2579 -> 2605, 128 2580 -> 2630.
+size_t skinny_columns(size_t in) { return in <= 768 ? 160 : 64; }
+
+// Whether a linear by itself takes the few-column kernel: the same limit (a
+// 1024-wide forward at 96 columns with its linears here one by one: 2594 -> 2998).
 bool skinny_fits(size_t in, size_t out, size_t cols, const float *w, const float *x) {
-  return cols <= 256 && in % 4 == 0 && in > 0 && in <= (size_t)INT32_MAX / 4 &&
+  return cols <= skinny_columns(in) && in % 4 == 0 && in > 0 && in <= (size_t)INT32_MAX / 4 &&
          out <= (size_t)INT32_MAX / 4 && aligned16(w) && aligned16(x);
 }
 
@@ -1200,7 +1209,7 @@ int laya_forward(tfd_ctx *c, const tfd_laya_model *m, const int64_t *ids, const 
   // Short batches: LayerNorm, the column moves around attention, GeGLU and
   // the residual adds inside the few-column linears, four launches and the
   // attention per layer instead of ten.
-  bool small = Tc <= 256 && d % 4 == 0 && d <= (size_t)tfd::kSkinnyNormMax && I % 4 == 0;
+  bool small = Tc <= skinny_columns(d) && d % 4 == 0 && d <= (size_t)tfd::kSkinnyNormMax && I % 4 == 0;
   for (size_t i = 0; i < m->n_layers; ++i) {
     const tfd_laya_encoder_layer &l = m->layers[i];
     for (const float *p : {l.attn_norm_w, l.attn_norm_b, l.wqkv, l.wo, l.mlp_norm_w, l.mlp_norm_b,
