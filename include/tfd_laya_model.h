@@ -7,7 +7,8 @@
  *        crates/laya-infer/tests/native_fixture.rs:75-139 checks against
  *        fixtures/laya-tiny/reference.json.
  *
- * Every linear runs as an f32 GEMM (rocBLAS), every attention block through
+ * Every linear is f32 (hand-written kernels; rocBLAS in between their size
+ * ranges and for unaligned weights), every attention block through
  * the fused split + RoPE + attention op of tfd_attention.h (structured
  * masks, build_mask semantics, model.rs:467-490), LayerNorm / GeGLU /
  * activations / pooling in small HIP kernels, all on the context's stream.
