@@ -19,15 +19,20 @@
 // per CU) keep the per-tile critical path short and the work per CU even
 // when rows differ in length.
 //
-// The products of the aligned path (VEC) run on the fp16 matrix cores, each
-// f32 operand as hi + lo fp16 scaled by a power of two, hi*hi + hi*lo + lo*hi
-// into f32: 24 16x16x32 instructions (384 cycles) per wave and tile instead
-// of 64 16x16x4 ones in f32 (2,048 cycles), which also kept the vector ALU idle
-// (f32 MFMAs and vector instructions of a SIMD never overlap; fp16 ones do).
-// Measured: L 512 B 8 (padded) 42.5 -> 29.7 us, L 2048 B 4 within +-64 51.4 -> 37 us
-// per call; relative error against 64 bits 2.6e-7 -> 2.0e-7 and 3.4e-7 -> 2.6e-7. Per
-// wave and tile about 180 vector instructions (half of them the split of K
-// and V), the LDS reads and the MFMAs follow one another and bound it together.
+// The products of the aligned path (VEC) run on the bf16 matrix cores, each f32
+// operand as three bf16 (split_bf16x3) and six products into f32: 48 16x16x32
+// instructions (768 cycles) per wave and tile instead of 64 16x16x4 ones in f32
+// (2,048 cycles), which also keep the vector ALU idle (f32 MFMAs and vector
+// instructions of a SIMD never overlap; bf16 ones do). The pieces hold all 24
+// bits over f32's whole exponent range and a key's depend on nothing but that key,
+// so a masked key's values, however large, never reach a query that does not keep it.
+// Pairs of fp16 with a scale per tile need half the products, but lose the kept
+// keys' bits beside a large key or feature. Measured (f32 MFMA -> fp16 pairs ->
+// this, us per call): L 512 B 8 (padded) 42.3 -> 29.7 -> 32.7, L 2048 B 4 within
+// +-64 51.2 -> 37.4 -> 40.2, L 395 B 3 24.7 -> 20.8 -> 20.3; relative error against 64
+// bits at L 512 2.6e-7 -> 2.0e-7 -> 1.0e-7. Per wave and tile about 230 vector
+// instructions (half of them the split of K and V), the LDS reads and the MFMAs
+// follow one another and bound it together.
 #include <type_traits>
 
 #include "tfd_device.hpp"
@@ -230,9 +235,9 @@ __device__ __forceinline__ f32x4 rot_hi(f32x4 x, f32x4 y, f32x4 c, f32x4 s) {
 // 2 GiB): buffer loads; a K task is one (key, chunk c) with its RoPE partner
 // chunk c + half/4 (and, with ROPE, the table chunks); a V task is one
 // feature of four consecutive keys, four 4-byte loads (a wave reads whole
-// key rows). Keys at or past L read as 0. The commit scales K and V by powers
-// of two, splits every element into hi + lo fp16 and writes both planes in the
-// order the 16x16x32 matrix cores read them: K as blocks of 16 keys x 32
+// key rows). Keys at or past L read as 0. The commit splits every element into
+// three bf16 (split_bf16x3) and writes the three planes of a block (1 KB each)
+// in the order the 16x16x32 matrix cores read them: K as blocks of 16 keys x 32
 // features, slot 16 * (feature / 8) + (key ^ 4 * (feature / 8)) of 16 bytes
 // (the exclusive or spreads one key's pieces over the banks), V as blocks of
 // 16 features, slot 16 * g + feature holding keys 4g .. 4g + 3 and 16 + 4g ..
@@ -245,8 +250,9 @@ template <int HDP, bool VEC, bool ROPE, int NT = 256>  // NT: threads that stage
 struct LayaStage {
   static constexpr int KS = HDP + 4;        // conflict-free 16-byte row reads
   static constexpr int VS = kKeyTile + 4;   // 16 lanes of 16-byte row pieces: conflict-free
-  static constexpr int KBUF = VEC ? kKeyTile * HDP : kKeyTile * KS;  // floats
-  static constexpr int VBUF = VEC ? kKeyTile * HDP : HDP * VS;
+  static constexpr int PB = 3 * 1024;       // bytes of a block's planes
+  static constexpr int KBUF = VEC ? kKeyTile * HDP * 3 / 2 : kKeyTile * KS;  // floats
+  static constexpr int VBUF = VEC ? kKeyTile * HDP * 3 / 2 : HDP * VS;
   static constexpr int KTASKS = kKeyTile * HDP / 8;
   static constexpr int VTASKS = (kKeyTile / 4) * HDP;
   static constexpr int KN = VEC ? (KTASKS + NT - 1) / NT : 1;
@@ -306,57 +312,34 @@ struct LayaStage {
     }
   }
 
-  // Rotates the fetched K in place (VEC).
-  __device__ __forceinline__ void rotate() {
-    if constexpr (ROPE) {
+  // Rotates the fetched K (VEC) and splits it and V.
+  Bf16x3 kp[VEC ? 2 * KN : 1], vp[VEC ? VN : 1];
+  __device__ __forceinline__ void split() {
 #pragma unroll
-      for (int i = 0; i < KN; ++i) {
-        const f32x4 lo = rot_lo(ka[i], kb[i], c[i], s[i]);
-        kb[i] = rot_hi(ka[i], kb[i], c[i], s[i]);
-        ka[i] = lo;
+    for (int i = 0; i < KN; ++i) {
+      f32x4 lo = ka[i], hi = kb[i];
+      if constexpr (ROPE) {
+        lo = rot_lo(ka[i], kb[i], c[i], s[i]);
+        hi = rot_hi(ka[i], kb[i], c[i], s[i]);
       }
+      kp[2 * i] = split_bf16x3(lo);
+      kp[2 * i + 1] = split_bf16x3(hi);
     }
+#pragma unroll
+    for (int i = 0; i < VN; ++i) vp[i] = split_bf16x3(v[i]);
   }
 
-  // This lane's largest magnitudes of the rotated K and of V (VEC).
-  __device__ __forceinline__ void lane_max(float &km, float &vm) const {
-    km = vm = 0.0f;
-#pragma unroll
-    for (int i = 0; i < KN; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) km = fmaxf(fmaxf(km, fabsf(ka[i][e])), fabsf(kb[i][e]));
-#pragma unroll
-    for (int i = 0; i < VN; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) vm = fmaxf(vm, fabsf(v[i][e]));
-  }
-  // The same over its finite elements.
-  __device__ __forceinline__ void lane_max_finite(float &km, float &vm) const {
-    km = vm = 0.0f;
-    auto fin = [](float x) { return __builtin_isfinite(x) ? fabsf(x) : 0.0f; };
-#pragma unroll
-    for (int i = 0; i < KN; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) km = fmaxf(fmaxf(km, fin(ka[i][e])), fin(kb[i][e]));
-#pragma unroll
-    for (int i = 0; i < VN; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) vm = fmaxf(vm, fin(v[i][e]));
-  }
-
-  // Writes the planes of the (rotated) tile times ksc and vsc (VEC).
-  __device__ __forceinline__ void write(int tid, float ksc, float vsc, float *Ks, float *Vs) const {
+  // Writes the planes of the split tile (VEC).
+  __device__ __forceinline__ void write(int tid, float *Ks, float *Vs) const {
     unsigned char *Kb = reinterpret_cast<unsigned char *>(Ks);
     unsigned char *Vb = reinterpret_cast<unsigned char *>(Vs);
-    auto put = [](unsigned char *p, f32x4 x, float scale) {
-      f16x4 hi, lo;
-      split_f16(x, scale, hi, lo);
-      *reinterpret_cast<f16x4 *>(p) = hi;
-      *reinterpret_cast<f16x4 *>(p + 1024) = lo;
+    auto put = [](unsigned char *p, const Bf16x3 &x) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x2 *>(p + 1024 * i) = x.p[i];
     };
     auto kslot = [&](int kk, int d) {
       const int oct = (d & 31) / 8;
-      return Kb + ((kk / 16) * (HDP / 32) + d / 32) * 2048 +
+      return Kb + ((kk / 16) * (HDP / 32) + d / 32) * PB +
              (oct * 16 + ((kk & 15) ^ (4 * oct))) * 16 + (d & 4) * 2;
     };
 #pragma unroll
@@ -364,8 +347,8 @@ struct LayaStage {
       const int task = tid + NT * i;
       if (KTASKS % NT == 0 || task < KTASKS) {
         const int kk = task / (HDP / 8), cp = task % (HDP / 8);
-        put(kslot(kk, 4 * cp), ka[i], ksc);
-        put(kslot(kk, HDP / 2 + 4 * cp), kb[i], ksc);
+        put(kslot(kk, 4 * cp), kp[2 * i]);
+        put(kslot(kk, HDP / 2 + 4 * cp), kp[2 * i + 1]);
       }
     }
 #pragma unroll
@@ -373,7 +356,7 @@ struct LayaStage {
       const int task = tid + NT * i;
       if (VTASKS % NT == 0 || task < VTASKS) {
         const int dd = task % HDP, kq = task / HDP;
-        put(Vb + (dd / 16) * 2048 + ((kq & 3) * 16 + (dd & 15)) * 16 + (kq >> 2) * 8, v[i], vsc);
+        put(Vb + (dd / 16) * PB + ((kq & 3) * 16 + (dd & 15)) * 16 + (kq >> 2) * 8, vp[i]);
       }
     }
   }
@@ -397,31 +380,6 @@ struct LayaStage {
       Vs[dd * VS + kk] = vv;
     }
   }
-};
-
-// Scales of a team's fp16 K/V tiles (VEC): x * 2^-e is stored, e taken from a
-// tile's largest magnitude so that it becomes [2^8, 2^9). A later tile keeps
-// e while its largest magnitude stays below fp16's range (2^15 scaled) and
-// above 2^2 scaled; otherwise e is taken anew for it. So an element keeps 22
-// bits, or an error of 2^-25 / 2^2 of its tile's largest if that is more.
-struct TileScale {
-  int ek = 0, ev = 0;
-  static __device__ __forceinline__ int exp_of(float mx, int keep) {
-    if (!(mx > 0.0f)) return keep;  // an all-zero tile fits any scale
-    const int e = (int)(__float_as_uint(mx) >> 23) - 126 - 9;  // denormals: -135, clamped
-    return max(-126, min(e, 126));
-  }
-  // A wave's word for a tile: bit 0 some element is past the range, bits 1
-  // and 2 some element of K, of V is above the lower bound.
-  __device__ __forceinline__ uint32_t word(float km, float vm) const {
-    // 2^(e + 15) and 2^(e + 2) as bits, ordered as the magnitudes are.
-    const uint32_t kb = __float_as_uint(km), vb = __float_as_uint(vm);
-    const uint32_t kh = (uint32_t)(ek + 142) << 23, vh = (uint32_t)(ev + 142) << 23;
-    const uint32_t kl = (uint32_t)(ek + 129) << 23, vl = (uint32_t)(ev + 129) << 23;
-    return ((__ballot(kb >= kh) | __ballot(vb >= vh)) != 0 ? 1u : 0u) |
-           (__ballot(kb >= kl) != 0 ? 2u : 0u) | (__ballot(vb >= vl) != 0 ? 4u : 0u);
-  }
-  static constexpr uint32_t kFine = 6u;
 };
 
 // ------------------------------------------------------------------- kernel
@@ -544,11 +502,12 @@ __device__ __noinline__ void laya_redo_wave(const LayaArgs *ap, int b, int head,
   }
 }
 
-// Occupancy target (laya_groups_per_cu): four workgroups (16 waves) per CU
-// where LDS and registers allow it (two per CU measured 41 us against 30 at L
-// 512 B 8): a wave's LDS reads, products and vector work follow one another,
-// so other waves have to cover them. For the same reason a second tile in
-// flight (two register stages, three workgroups per CU) was slower, 38 us.
+// Occupancy target (laya_groups_per_cu): as many workgroups per CU as the walk's
+// registers allow without spilling. At hd 64 that is three, with operands read
+// a step ahead of their products: four at 128 registers spilled inside the walk, and
+// waiting for a spilled register also waits for the next tile's loads (44 us
+// against 34 at L 512 B 8). Two K/V buffers instead of one with two barriers
+// per tile: 34.2 -> 32.7 us. V's first operands read before the exponentials: 33.8.
 template <int HDP, int MODE, bool VEC, bool ROPE, bool VW, int TEAMS, int QW>
 __global__ __launch_bounds__(64 * QW * TEAMS, TEAMS == 1 ? laya_groups_per_cu(HDP) : 1) void laya_attention_kernel(
     const LayaArgs a) {
@@ -557,24 +516,23 @@ __global__ __launch_bounds__(64 * QW * TEAMS, TEAMS == 1 ? laya_groups_per_cu(HD
   using Stage = LayaStage<HDP, VEC, ROPE, NT>;
   constexpr int KS = Stage::KS, VS = Stage::VS;
   constexpr int QS = HDP / 4;   // Q elements per lane (4 lane groups split hd)
-  constexpr int K32 = HDP / 32; // 32-feature steps of the fp16 products
+  constexpr int K32 = HDP / 32; // 32-feature steps of the bf16 products
   constexpr int NB = HDP / 16;  // 16-row blocks of O^T
   constexpr int GQ = kLayaWaveQueries * QW;  // queries per workgroup
   // TEAMS > 1 (grids of at most one workgroup per CU): TEAMS teams of four
   // waves, each with its own K/V buffers, walk every TEAMS-th key tile of
   // the workgroup's span and merge their (m, l, O) once at the end.
-  constexpr int TB = 2 * (Stage::KBUF + Stage::VBUF);  // floats per team
-  constexpr int NWAVES = TEAMS * QW;
+  // Two K/V buffers per team where the CU's LDS holds them for all its
+  // workgroups (always without VEC), else one.
+  constexpr int BUF = Stage::KBUF + Stage::VBUF;  // floats
+  constexpr bool TWO = !VEC || 2 * BUF * 4 * TEAMS * (TEAMS == 1 ? laya_groups_per_cu(HDP) : 1) <= 155648;
+  constexpr int TB = (TWO ? 2 : 1) * BUF;  // floats per team
   static_assert(TEAMS == 1 || (TEAMS - 1) * 4 * (4 * (HDP / 16) + 2) * 64 + 4 * kKeyTile * 17 <= TEAMS * TB,
                 "merge data and the redo rows fit in the teams' K/V buffers");
   __shared__ __attribute__((aligned(16))) float smem[TEAMS * TB];
   const int team = TEAMS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT);
-  auto Ks = [&](int i) { return smem + team * TB + i * (Stage::KBUF + Stage::VBUF); };
+  auto Ks = [&](int i) { return smem + team * TB + (TWO ? i * BUF : 0); };
   auto Vs = [&](int i) { return Ks(i) + Stage::KBUF; };
-  // VEC: the waves' largest K and V magnitudes where the tile scales are taken
-  // anew, and their words for the tile in each buffer.
-  __shared__ float s_amax[VEC ? 2 * NWAVES : 1];
-  __shared__ __attribute__((aligned(16))) uint32_t s_word[VEC ? 2 * NWAVES : 1];
 
   const int tid = TEAMS == 1 ? (int)threadIdx.x : (int)(threadIdx.x & (NT - 1)), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform, in a scalar register
@@ -665,19 +623,18 @@ __global__ __launch_bounds__(64 * QW * TEAMS, TEAMS == 1 ? laya_groups_per_cu(HD
 
   // -------- Q: rotated, in registers. !VEC: lane (col, grp) holds
   // Q[q][grp*QS + x] for x < QS, the B operand of step x. VEC: Q[q][32*s +
-  // 8*grp + e] as hi + lo fp16 of Q * 2^-eq, eq of the query's largest
-  // magnitude; the scores come back through the query's c1 * 2^(eq + ek).
+  // 8*grp + e] as three bf16.
   float qreg[VEC ? 1 : QS];
-  f16x8 qh[VEC ? K32 : 1], ql[VEC ? K32 : 1];
+  bf16x8 qp[3][VEC ? K32 : 1];
   const int qq = qin ? q : 0;
   const int d0 = grp * QS;
   // VEC (hd == HDP): the wave's 16 Q rows are loaded along the rows, so that
   // every load instruction reads whole cache lines once: task (t, p) is
   // token q0w + t with its chunk pair (p, p + hd/8), the two 16-byte pieces
   // that RoPE rotates together, plus table chunk p of that token. The
-  // rotated rows go to the wave's staging rows in LDS (the second K/V
-  // buffer, unused until the walk's first barrier has passed) and come back
-  // in the MFMA layout after the loads.
+  // rotated rows go to the wave's staging rows in LDS (the last K/V buffer:
+  // the second is unused until the walk's first barrier has passed) and come
+  // back in the MFMA layout after the loads.
   constexpr int QT = 16 * HDP / 8 / 64;  // tasks per lane
   f32x4 qlo4[VEC ? QT : 1], qhi4[VEC ? QT : 1], qc4[VEC && ROPE ? QT : 1], qs4[VEC && ROPE ? QT : 1];
   float *qst = nullptr;
@@ -685,7 +642,7 @@ __global__ __launch_bounds__(64 * QW * TEAMS, TEAMS == 1 ? laya_groups_per_cu(HD
   auto qchunk = [&](int t, int c) { return qst + t * HDP + 4 * (c ^ (t & (HDP / 4 - 1))); };
   if constexpr (VEC) {
     static_assert(QW * 16 * HDP <= Stage::KBUF + Stage::VBUF,
-                  "the team's Q rows fit in its second K/V buffer");
+                  "the team's Q rows fit in its last K/V buffer");
     qst = Ks(1) + wave * 16 * HDP;
 #pragma unroll
     for (int i = 0; i < QT; ++i) {
@@ -839,7 +796,6 @@ __global__ __launch_bounds__(64 * QW * TEAMS, TEAMS == 1 ? laya_groups_per_cu(HD
     }
   }
 
-  float c1q = a.c1;  // scores to the log2 domain (VEC: of this query's scaled Q)
   if constexpr (VEC) {
 #pragma unroll
     for (int i = 0; i < QT; ++i) {
@@ -855,29 +811,18 @@ __global__ __launch_bounds__(64 * QW * TEAMS, TEAMS == 1 ? laya_groups_per_cu(HD
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    f32x4 qv[2 * K32];
-    float mx = 0.0f;
 #pragma unroll
-    for (int c = 0; c < 2 * K32; ++c) {
-      qv[c] = *reinterpret_cast<const f32x4 *>(qchunk(col, 8 * (c / 2) + 2 * grp + (c & 1)));
+    for (int x = 0; x < K32; ++x) {
+      f32x4 v[2];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        qv[c][e] = qin ? qv[c][e] : 0.0f;
-        mx = fmaxf(mx, __builtin_isfinite(qv[c][e]) ? fabsf(qv[c][e]) : 0.0f);
+      for (int c = 0; c < 2; ++c) {
+        v[c] = *reinterpret_cast<const f32x4 *>(qchunk(col, 8 * x + 2 * grp + c));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[c][e] = qin ? v[c][e] : 0.0f;
       }
-    }
-    mx = pair_max(pair16_max(mx));
-    const int eq = TileScale::exp_of(mx, 0);
-    c1q = ldexpf(a.c1, eq);
+      const Bf16x3 lo = split_bf16x3(v[0]), hi = split_bf16x3(v[1]);
 #pragma unroll
-    for (int c = 0; c < 2 * K32; ++c) {
-      f16x4 hi, lo;
-      split_f16(qv[c], pow2i(-eq), hi, lo);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        qh[c / 2][4 * (c & 1) + e] = hi[e];
-        ql[c / 2][4 * (c & 1) + e] = lo[e];
-      }
+      for (int i = 0; i < 3; ++i) qp[i][x] = join_bf16(lo, hi, i);
     }
   } else {
     const float *row = xb + (size_t)qq * tok;
@@ -926,45 +871,19 @@ __global__ __launch_bounds__(64 * QW * TEAMS, TEAMS == 1 ? laya_groups_per_cu(HD
     for (int r = 0; r < 4; ++r) O[j][r] = 0.0f;
   float m = kNoMax, l = 0.0f;  // l: this lane's share of the row sum
 
-  // VEC: takes the scales of the tile in `st` from its largest magnitudes
-  // over the team's waves and writes its planes to buffer `buf`; every wave
-  // of the workgroup calls it (have: its team has a tile). One barrier inside;
-  // the caller's next one publishes the planes.
-  TileScale sc;
-  auto rescale_tile = [&](bool have, bool take, int buf) {
-    float km = 0.0f, vm = 0.0f;
-    if (have) st.lane_max_finite(km, vm);
-    km = wave_max_f(km);
-    vm = wave_max_f(vm);
-    if (lane == 0) {
-      s_amax[2 * (team * QW + wave)] = km;
-      s_amax[2 * (team * QW + wave) + 1] = vm;
-    }
-    __syncthreads();
-    if (have && take) {
-#pragma unroll
-      for (int i = 0; i < QW; ++i) {
-        km = fmaxf(km, s_amax[2 * (team * QW + i)]);
-        vm = fmaxf(vm, s_amax[2 * (team * QW + i) + 1]);
-      }
-      sc.ek = __builtin_amdgcn_readfirstlane(TileScale::exp_of(km, sc.ek));
-      sc.ev = __builtin_amdgcn_readfirstlane(TileScale::exp_of(vm, sc.ev));
-    }
-    if (have) st.write(tid, pow2i(-sc.ek), pow2i(-sc.ev), Ks(buf), Vs(buf));
-    if (lane == 0) s_word[buf * NWAVES + team * QW + wave] = TileScale::kFine;
-  };
   auto first_tile = [&]() {
     if constexpr (VEC) {
-      if (tb < te) st.rotate();
-      rescale_tile(tb < te, true, 0);
+      if (tb < te) st.split();
+      if constexpr (!TWO) __syncthreads();  // every wave has read its Q rows back
+      if (tb < te) st.write(tid, Ks(0), Vs(0));
     } else if (tb < te) {
       st.commit(a, xb, tok, tb * kKeyTile, tid, Ks(0), Vs(0));
     }
   };
 
   // -------- the walk: tile kt+1 is fetched into registers before the
-  // products of tile kt and committed to the other LDS buffer after them;
-  // one barrier per tile. A 32-key tile is two S^T blocks: s0 holds keys
+  // products of tile kt and committed to the other LDS buffer after them, one
+  // barrier per tile (one buffer: between two barriers). A 32-key tile is two S^T blocks: s0 holds keys
   // 4*grp + r, s1 keys 16 + 4*grp + r of query col.
   //
   // Exponents are exp2(fma(s, c1, -m)) against a reference m (log2 units)
@@ -1013,11 +932,7 @@ __global__ __launch_bounds__(64 * QW * TEAMS, TEAMS == 1 ? laya_groups_per_cu(HD
   __builtin_amdgcn_s_waitcnt(0);
   bool tainted = false;  // wave-uniform
   int cur = 0;
-  // VEC: probabilities are taken 2^kShift times larger, so that as fp16 pairs
-  // they keep an absolute error of 2^-25 / 2^kShift of the row's largest; they
-  // stay below 2^(kShift + kRescaleSlack) = 2^15, fp16's range.
-  constexpr float kShift = VEC ? 7.0f : 0.0f;
-  constexpr float kLimit = VEC ? 32768.0f : kLazyLimit;
+  const float c1 = a.c1;
   for (int kt = tb; kt < kt_stop; kt += TEAMS) {
     const bool act = TEAMS == 1 || kt < te;  // a team with fewer tiles idles at its last step
     const bool more = kt + TEAMS < te;
@@ -1025,27 +940,40 @@ __global__ __launch_bounds__(64 * QW * TEAMS, TEAMS == 1 ? laya_groups_per_cu(HD
       m_next = mask_of(kt + TEAMS);
       st.fetch((kt + TEAMS) * kKeyTile);
     }
-    const bool mine = act && !tainted && __ballot(w != 0u) != 0;  // wave-uniform
-    f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = {0.0f, 0.0f, 0.0f, 0.0f};
-    // S^T: K from LDS against the Q registers, two independent chains.
-    auto scores = [&]() {
-      s0 = s1 = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (act && !tainted && __ballot(w != 0u) != 0) {  // wave-uniform
+      // S^T: K from LDS against the Q registers, two independent chains.
+      f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = {0.0f, 0.0f, 0.0f, 0.0f};
       if constexpr (VEC) {
         const unsigned char *Kc = reinterpret_cast<const unsigned char *>(Ks(cur)) +
                                   (grp * 16 + (col ^ (4 * grp))) * 16;
+        // The products but h*h (2^-8 of the sum) have accumulators of their own:
+        // the matrix cores round the sum once per instruction.
+        // Operands one step ahead of their products.
+        f32x4 r0 = s0, r1 = s1;
+        bf16x8 k[2][6];
+        auto take = [&](int x) {
+#pragma unroll
+          for (int i = 0; i < 6; ++i)
+            k[x & 1][i] = *reinterpret_cast<const bf16x8 *>(
+                Kc + Stage::PB * (K32 * (i / 3) + x) + 1024 * (i % 3));
+        };
+        take(0);
 #pragma unroll
         for (int x = 0; x < K32; ++x) {
-          const f16x8 k0h = *reinterpret_cast<const f16x8 *>(Kc + 2048 * x);
-          const f16x8 k0l = *reinterpret_cast<const f16x8 *>(Kc + 2048 * x + 1024);
-          const f16x8 k1h = *reinterpret_cast<const f16x8 *>(Kc + 2048 * (K32 + x));
-          const f16x8 k1l = *reinterpret_cast<const f16x8 *>(Kc + 2048 * (K32 + x) + 1024);
-          s0 = mfma_16x16x32_f16(k0h, ql[x], s0);
-          s1 = mfma_16x16x32_f16(k1h, ql[x], s1);
-          s0 = mfma_16x16x32_f16(k0l, qh[x], s0);
-          s1 = mfma_16x16x32_f16(k1l, qh[x], s1);
-          s0 = mfma_16x16x32_f16(k0h, qh[x], s0);
-          s1 = mfma_16x16x32_f16(k1h, qh[x], s1);
+          if (x + 1 < K32) take(x + 1);
+          const bf16x8 (&kx)[6] = k[x & 1];
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; i + j < 3; ++j) {
+              f32x4 &t0 = i + j ? r0 : s0, &t1 = i + j ? r1 : s1;
+              t0 = mfma_16x16x32_bf16(kx[i], qp[j][x], t0);
+              t1 = mfma_16x16x32_bf16(kx[3 + i], qp[j][x], t1);
+            }
+          __builtin_amdgcn_sched_barrier(0);
         }
+        s0 += r0;
+        s1 += r1;
       } else {
         const float *Kc = Ks(cur);
         const f32x4 *k0p = reinterpret_cast<const f32x4 *>(&Kc[col * KS + d0]);
@@ -1060,50 +988,13 @@ __global__ __launch_bounds__(64 * QW * TEAMS, TEAMS == 1 ? laya_groups_per_cu(HD
           }
         }
       }
-    };
-    uint32_t words = 0u, fine = 1u;
-    if constexpr (VEC) {
-#pragma unroll
-      for (int i = 0; i < NWAVES; i += QW) {  // per team: no range error, both above the bound
-        words = 0u;
-#pragma unroll
-        for (int j = 0; j < QW; ++j) words |= s_word[cur * NWAVES + i + j];
-        fine &= words == TileScale::kFine ? 1u : 0u;
-      }
-    }
-    if (mine) scores();
-    if constexpr (VEC) {
-      if (__builtin_amdgcn_readfirstlane(fine) == 0u) {
-        // Rare: some team's tile does not fit its scales. Every team takes
-        // part in the barriers; one whose tile fits rewrites the same bits.
-        words = 0u;
-#pragma unroll
-        for (int j = 0; j < QW; ++j) words |= s_word[cur * NWAVES + team * QW + j];
-        const int ev = sc.ev;
-        if (act) {
-          st.fetch(kt * kKeyTile);
-          st.rotate();
-        }
-        __syncthreads();  // every wave has read the words and its operands
-        rescale_tile(act, __builtin_amdgcn_readfirstlane(words) != TileScale::kFine, cur);
-        __syncthreads();
-        if (more) st.fetch((kt + TEAMS) * kKeyTile);
-        const float f = ldexpf(1.0f, ev - sc.ev);  // O's unit is 2^ev
-        if (ev != sc.ev) {
-#pragma unroll
-          for (int j = 0; j < NB; ++j) O[j] *= f;
-        }
-        if (mine) scores();
-      }
-    }
-    const float c1 = VEC ? c1q * pow2i(sc.ek) : c1q;
-    if (mine) {
       if (__ballot(qin && w != 0xffffffffu) != 0) {
         // A tile some query of the wave keeps only in part: mask it.
+        const uint32_t wg = w >> (4 * grp);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          s0[r] = ((w >> (4 * grp + r)) & 1u) ? s0[r] : -INFINITY;
-          s1[r] = ((w >> (16 + 4 * grp + r)) & 1u) ? s1[r] : -INFINITY;
+          s0[r] = ((wg >> r) & 1u) ? s0[r] : -INFINITY;
+          s1[r] = ((wg >> (16 + r)) & 1u) ? s1[r] : -INFINITY;
         }
       }
       f32x4 e0, e1;
@@ -1115,14 +1006,14 @@ __global__ __launch_bounds__(64 * QW * TEAMS, TEAMS == 1 ? laya_groups_per_cu(HD
         rs += e0[r] + e1[r];
       }
       bool ok = true;
-      if (__ballot(qin && !(rs <= kLimit)) != 0) {
+      if (__ballot(qin && !(rs <= kLazyLimit)) != 0) {
         // Move the reference where the tile max exceeds it by more than the
         // slack (the first tile always: m starts at kNoMax).
         const float mx = fmaxf(fmaxf(fmaxf(s0[0], s0[1]), fmaxf(s0[2], s0[3])),
                                fmaxf(fmaxf(s1[0], s1[1]), fmaxf(s1[2], s1[3])));
         const float mxs = pair_max(pair16_max(mx)) * c1;
-        const bool need = mxs > m + (kRescaleSlack + kShift);
-        const float mn = need ? mxs - kShift : m;
+        const bool need = mxs > m + kRescaleSlack;
+        const float mn = need ? mxs : m;
         rs = 0.0f;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -1144,19 +1035,35 @@ __global__ __launch_bounds__(64 * QW * TEAMS, TEAMS == 1 ? laya_groups_per_cu(HD
       if (ok) {
         l += rs;
         if constexpr (VEC) {
-          f16x4 h0, l0, h1, l1;
-          split_f16(e0, h0, l0);
-          split_f16(e1, h1, l1);
-          const f16x8 ph = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
-          const f16x8 pl = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
-          const unsigned char *vp = reinterpret_cast<const unsigned char *>(Vs(cur)) + 16 * lane;
+          const Bf16x3 p0 = split_bf16x3(e0), p1 = split_bf16x3(e1);
+          bf16x8 pp[3];
 #pragma unroll
-          for (int j = 0; j < NB; ++j) {
-            const f16x8 vh = *reinterpret_cast<const f16x8 *>(vp + 2048 * j);
-            const f16x8 vl = *reinterpret_cast<const f16x8 *>(vp + 2048 * j + 1024);
-            O[j] = mfma_16x16x32_f16(vh, pl, O[j]);
-            O[j] = mfma_16x16x32_f16(vl, ph, O[j]);
-            O[j] = mfma_16x16x32_f16(vh, ph, O[j]);
+          for (int i = 0; i < 3; ++i) pp[i] = join_bf16(p0, p1, i);
+          const unsigned char *vc = reinterpret_cast<const unsigned char *>(Vs(cur)) + 16 * lane;
+          bf16x8 v[2][6];
+          auto take = [&](int j) {  // blocks j and j + 1
+#pragma unroll
+            for (int i = 0; i < 6; ++i)
+              v[(j / 2) & 1][i] = *reinterpret_cast<const bf16x8 *>(
+                  vc + Stage::PB * (j + i / 3) + 1024 * (i % 3));
+          };
+          take(0);
+#pragma unroll
+          for (int j = 0; j < NB; j += 2) {
+            if (j + 2 < NB) take(j + 2);
+            const bf16x8 (&vx)[6] = v[(j / 2) & 1];
+            f32x4 low0 = {0.0f, 0.0f, 0.0f, 0.0f}, low1 = low0;
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+              for (int x = 0; i + x < 3; ++x) {
+                f32x4 &t0 = i + x ? low0 : O[j], &t1 = i + x ? low1 : O[j + 1];
+                t0 = mfma_16x16x32_bf16(vx[i], pp[x], t0);
+                t1 = mfma_16x16x32_bf16(vx[3 + i], pp[x], t1);
+              }
+            O[j] += low0;
+            O[j + 1] += low1;
+            __builtin_amdgcn_sched_barrier(0);
           }
         } else {
           // A operand of block j: V[key 4*grp + r (+16)][d = 16*j + col], one
@@ -1175,15 +1082,9 @@ __global__ __launch_bounds__(64 * QW * TEAMS, TEAMS == 1 ? laya_groups_per_cu(HD
       }
     }
     if constexpr (VEC) {
-      uint32_t word = TileScale::kFine;
-      if (more) {
-        float km, vm;
-        st.rotate();
-        st.lane_max(km, vm);
-        word = sc.word(km, vm);
-        st.write(tid, pow2i(-sc.ek), pow2i(-sc.ev), Ks(cur ^ 1), Vs(cur ^ 1));
-      }
-      if (lane == 0) s_word[(cur ^ 1) * NWAVES + team * QW + wave] = word;
+      if (more) st.split();
+      if constexpr (!TWO) __syncthreads();  // every wave has read the tile
+      if (more) st.write(tid, Ks(cur ^ 1), Vs(cur ^ 1));
     } else if (more) {
       st.commit(a, xb, tok, (kt + TEAMS) * kKeyTile, tid, Ks(cur ^ 1), Vs(cur ^ 1));
     }
@@ -1195,11 +1096,6 @@ __global__ __launch_bounds__(64 * QW * TEAMS, TEAMS == 1 ? laya_groups_per_cu(HD
   // -------- careful redo (rare): NaN / inf among this wave's kept scores
   // or values. Every wave's LDS reads of the walk precede its last barrier,
   // so the wave may now use its own slice of the LDS block.
-  if constexpr (VEC) {
-    const float f = pow2i(sc.ev);
-#pragma unroll
-    for (int j = 0; j < NB; ++j) O[j] *= f;
-  }
   bool bad = false;
 #pragma unroll
   for (int j = 0; j < NB; ++j)
@@ -1374,11 +1270,11 @@ static hipError_t launch_laya_hd(const LayaArgs &a, int heads, int batch, int mo
     return hipErrorInvalidValue;
   if (a.cus > 0 && a.nkt > 1 && groups * 2 <= a.cus) {
     const dim3 grid((a.L + 2 * kLayaWaveQueries - 1) / (2 * kLayaWaveQueries), heads, batch);
-    return launch_laya_teams<HDP, VEC, ROPE, laya_teams(HDP), 2>(a, grid, mode, stream, ev);
+    return launch_laya_teams<HDP, VEC, ROPE, laya_teams(HDP, 2), 2>(a, grid, mode, stream, ev);
   }
   const dim3 grid(ng, heads, batch);
   if (laya_teams_grid(a.L, heads, batch, a.nkt, a.cus))
-    return launch_laya_teams<HDP, VEC, ROPE, laya_teams(HDP), 4>(a, grid, mode, stream, ev);
+    return launch_laya_teams<HDP, VEC, ROPE, laya_teams(HDP, 4), 4>(a, grid, mode, stream, ev);
   LayaArgs b = a;
   b.layout = 0;
   if (laya_xcd_layout((int)ng, heads, batch, laya_groups_per_cu(HDP), a.cus))

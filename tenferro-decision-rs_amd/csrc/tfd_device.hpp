@@ -9,6 +9,8 @@ namespace tfd {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
@@ -214,6 +216,37 @@ __device__ __forceinline__ int norm_weight_exp(const float *__restrict__ w, int 
 __device__ __forceinline__ unsigned short f32_to_f16_bits(float x) {
   const _Float16 h = (_Float16)x;
   return __builtin_bit_cast(unsigned short, h);
+}
+
+// f32 operands on the bf16 matrix cores: v = h + m + l, each the bf16 nearest to
+// what the ones before leave (24 significant bits in three times eight, so
+// the sum is v itself down to |v| = 2^-110, below it v to 2^-134). bf16 has
+// f32's exponent range: no scale, and no element's pieces depend on another
+// element. A product v * w is taken as hh' + (hm' + mh') + (hl' + lh' + mm'); the
+// dropped ml', lm' and ll' are below 2^-24 of |v w|, f32's own rounding. inf and NaN
+// (and finite values that round to inf in bf16) give pieces that are inf or NaN.
+// 22 vector instructions for four elements.
+struct Bf16x3 {
+  u32x2 p[3];
+};
+__device__ __forceinline__ Bf16x3 split_bf16x3(f32x4 v) {
+  Bf16x3 s;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    s.p[i] = __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
+    if (i < 2) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t w = s.p[i][e >> 1];
+        v[e] -= __uint_as_float((e & 1) ? (w & 0xffff0000u) : (w << 16));
+      }
+    }
+  }
+  return s;
+}
+// Piece i of eight consecutive elements, split as lo and hi four.
+__device__ __forceinline__ bf16x8 join_bf16(const Bf16x3 &lo, const Bf16x3 &hi, int i) {
+  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo.p[i], hi.p[i], 0, 1, 2, 3));
 }
 
 // v * scale (a power of two) as hi + lo fp16: hi = fp16(v), lo = fp16(v -

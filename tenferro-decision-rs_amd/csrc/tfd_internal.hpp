@@ -22,14 +22,19 @@ constexpr int kJeffKeyTile = 16;      // keys per Jeff f32 tile
 // whole 64-byte scalar loads.
 __host__ __device__ constexpr int laya_map_row(int nkt) { return (nkt + 63) & ~63; }
 
-// Laya workgroups per CU (launch bounds): four at padded head dims up to 64,
-// two at 128.
-__host__ __device__ constexpr int laya_groups_per_cu(int hd_pad) { return hd_pad <= 64 ? 4 : 2; }
+// Laya workgroups per CU (launch bounds), by the walk's registers: four at
+// padded head dim 32 (128 of them), three at 64 (168), two at 128 (256).
+__host__ __device__ constexpr int laya_groups_per_cu(int hd_pad) {
+  return hd_pad <= 32 ? 4 : (hd_pad <= 64 ? 3 : 2);
+}
 
-// Teams of four waves per Laya workgroup when the grid has at most one
-// workgroup per CU: as many as the teams' double-buffered K/V tiles fit in a
-// CU's LDS (four at padded head dims up to 64, two at 128).
-__host__ __device__ constexpr int laya_teams(int hd_pad) { return hd_pad <= 64 ? 4 : 2; }
+// Teams of `waves` waves per Laya workgroup when the grid has at most one
+// workgroup per CU: as many as the same registers and the teams' K/V tiles in
+// a CU's LDS allow (four-wave teams at 64: three, as four at 128 registers spill
+// and took 38 us instead of 21 at L 395 B 3).
+__host__ __device__ constexpr int laya_teams(int hd_pad, int waves) {
+  return hd_pad <= 32 ? 4 : (hd_pad <= 64 ? (waves == 4 ? 3 : 4) : 2);
+}
 
 // Whether a Laya grid of nqb x H x B workgroups gets the XCD-aware layout:
 // the whole grid fits in one dispatch round (workgroup p then runs on XCD
