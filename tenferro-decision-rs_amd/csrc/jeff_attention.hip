@@ -280,17 +280,22 @@ __global__ __launch_bounds__(256) void jeff_k_prep_kernel(const JeffArgs a, OutT
   }
 }
 
-// Planes of the f32 kernel at hd 256: per (row, kv head) and 32-key tile 64
-// KB in the order the 16x16x32 fp16 matrix cores read them, every f32 as hi +
-// lo fp16 (1 KB blocks, 16 bytes per lane, hi then lo). K: blocks (16-key half
-// b, step s), lane (key, g) holding features 32 s + 8 g .. + 7. V: blocks of 16
-// features, lane (feature, g) holding keys 4 g .. + 3 and 16 + 4 g .. + 3, the
-// keys whose probabilities lane group g of S^T holds.
-constexpr int kJeffTileBytes = 65536, kJeffTileV = 32768;
-// Normalized keys and queries times 2^(kJeffNormUp - e), e =
-// norm_weight_exp: below 2^14, so lo still holds elements 2^-24 of the largest
-// to 2^-11 of themselves.
-constexpr int kJeffNormUp = 10;
+// Planes of the f32 kernel at hd 256: per (row, kv head) and 32-key tile 96
+// KB in the order the 16x16x32 bf16 matrix cores read them, every f32 as three
+// bf16 (split_bf16x3; blocks of three 1 KB planes, 16 bytes per lane). K: blocks
+// (16-key half b, step s), lane (key, g) holding features 32 s + 8 g .. + 7. V:
+// blocks of 16 features, lane (feature, g) holding keys 4 g .. + 3 and 16 + 4 g
+// .. + 3, the keys whose probabilities lane group g of S^T holds. The attention
+// kernel walks a tile as four pieces: the K halves, then V's feature halves.
+constexpr int kJeffBlock = 3072, kJeffPieceBytes = 8 * kJeffBlock;
+constexpr int kJeffTileBytes = 4 * kJeffPieceBytes, kJeffTileV = 2 * kJeffPieceBytes;
+
+// Writes eight elements' planes (a lane's 16 bytes in each).
+__device__ __forceinline__ void write_planes(unsigned char *p, f32x4 lo, f32x4 hi) {
+  const Bf16x3 a = split_bf16x3(lo), b = split_bf16x3(hi);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8 *>(p + 1024 * i) = join_bf16(a, b, i);
+}
 
 // One workgroup = the K (blockIdx.y even) or V planes of one (row, kv head,
 // 32-key tile): the split done once per call instead of once per query tile
@@ -300,14 +305,12 @@ constexpr int kJeffNormUp = 10;
 // over the eight parts (lane swap, then LDS), partial RoPE (692-709) in
 // registers when the partner feature i + rot/2 sits in the same wave (rot/2 =
 // 32: part p pairs with part p + 1, lane + 32), else through LDS. V: thread =
-// feature, its 32 keys as eight 16-byte loads (dword alignment suffices),
-// scaled by 2^-e of the tile's largest magnitude (vexp). Workgroups with
-// blockIdx.x == 0 of kv head 0 also write the row's active-key bits and key
-// span, row 0's the norm exponents (spans[-2], spans[-1]). Bound by HBM and one
-// memory round trip.
+// feature, its 32 keys as eight 16-byte loads (dword alignment suffices).
+// Workgroups with blockIdx.x == 0 of kv head 0 also write the row's active-key
+// bits and key span. Bound by HBM and one memory round trip.
 __global__ __launch_bounds__(256) void jeff_k_prep_split_kernel(
-    const JeffArgs a, unsigned char *__restrict__ planes, int *__restrict__ vexp,
-    int *__restrict__ spans, uint32_t *__restrict__ kbits) {
+    const JeffArgs a, unsigned char *__restrict__ planes, int *__restrict__ spans,
+    uint32_t *__restrict__ kbits) {
   constexpr int HDP = 256, KB = 32, KS = HDP + 4;
   __shared__ __attribute__((aligned(16))) float Kt[KB * KS];
   __shared__ float s_red[4 * KB];
@@ -335,32 +338,14 @@ __global__ __launch_bounds__(256) void jeff_k_prep_split_kernel(
     f32x4 x[8];
 #pragma unroll
     for (int c = 0; c < 8; ++c) x[c] = buffer_load4(rv, (tid * L + 4 * c) * 4, k0 * 4);
-    float mx = 0.0f;
 #pragma unroll
     for (int c = 0; c < 8; ++c)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        // Past L lies the next feature; past hd the loads read 0.
+      for (int e = 0; e < 4; ++e)  // past L lies the next feature; past hd the loads read 0
         x[c][e] = k0 + 4 * c + e < L ? x[c][e] : 0.0f;
-        mx = fmaxf(mx, __builtin_isfinite(x[c][e]) ? fabsf(x[c][e]) : 0.0f);
-      }
-    mx = wave_max_f(mx);
-    if (lane == 0) s_red[wave] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
-    const int ev = max(-126, (int)(__float_as_uint(mx) >> 23) - 126 - 15);  // zero or denormal: -126
-    if (tid == 0) vexp[unit] = ev;
-    const float sc = pow2i(-ev);
-    unsigned char *p = tile + kJeffTileV + (tid >> 4) * 2048 + (tid & 15) * 16;
+    unsigned char *p = tile + kJeffTileV + (tid >> 4) * kJeffBlock + (tid & 15) * 16;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      f16x4 h0, l0, h1, l1;
-      split_f16(x[g], sc, h0, l0);
-      split_f16(x[4 + g], sc, h1, l1);
-      *reinterpret_cast<f16x8 *>(p + 256 * g) = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
-      *reinterpret_cast<f16x8 *>(p + 256 * g + 1024) =
-          __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
-    }
+    for (int g = 0; g < 4; ++g) write_planes(p + 256 * g, x[g], x[4 + g]);
     return;
   }
 
@@ -390,17 +375,7 @@ __global__ __launch_bounds__(256) void jeff_k_prep_split_kernel(
       ts[c] = *reinterpret_cast<const f32x4 *>(a.sin_t + pos + 4 * c);
     }
   }
-  const int ek = norm_weight_exp(a.k_norm, hd, lane);
-  if (blockIdx.x == 0 && kvh == 0 && wave == 0) {
-    write_row_bits_span(maskr, L, lane, row, spans, kbits);
-    if (row == 0) {  // the attention kernel's norm exponents
-      const int eq = norm_weight_exp(a.q_norm, hd, lane);
-      if (lane == 0) {
-        spans[-2] = eq;
-        spans[-1] = ek;
-      }
-    }
-  }
+  if (blockIdx.x == 0 && kvh == 0 && wave == 0) write_row_bits_span(maskr, L, lane, row, spans, kbits);
 
   float ss = 0.0f;
 #pragma unroll
@@ -450,16 +425,11 @@ __global__ __launch_bounds__(256) void jeff_k_prep_split_kernel(
 #pragma unroll
     for (int j = 0; j < 32; ++j) kv[j] = Kt[kk * KS + 32 * part + j];
   }
-  const float sc = pow2i(kJeffNormUp - ek);
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {  // step part, lane group c
-    f16x4 h0, l0, h1, l1;
-    split_f16(f32x4{kv[8 * c], kv[8 * c + 1], kv[8 * c + 2], kv[8 * c + 3]}, sc, h0, l0);
-    split_f16(f32x4{kv[8 * c + 4], kv[8 * c + 5], kv[8 * c + 6], kv[8 * c + 7]}, sc, h1, l1);
-    unsigned char *p = tile + ((kk >> 4) * 8 + part) * 2048 + (c * 16 + (kk & 15)) * 16;
-    *reinterpret_cast<f16x8 *>(p) = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
-    *reinterpret_cast<f16x8 *>(p + 1024) = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
-  }
+  for (int c = 0; c < 4; ++c)  // step part, lane group c
+    write_planes(tile + ((kk >> 4) * 8 + part) * kJeffBlock + (c * 16 + (kk & 15)) * 16,
+                 f32x4{kv[8 * c], kv[8 * c + 1], kv[8 * c + 2], kv[8 * c + 3]},
+                 f32x4{kv[8 * c + 4], kv[8 * c + 5], kv[8 * c + 6], kv[8 * c + 7]});
 }
 
 // ----------------------------------------------------------- f32 attention
@@ -1155,38 +1125,43 @@ __device__ __forceinline__ void jeff_unit_of(const JeffArgs &a, int rows, int u,
 
 // One workgroup = 4 wavefronts = hg query heads of a GQA group (hg = 4, 2 or
 // 1) x 4 / hg query tiles of 16; a wave owns one head's 16 queries and walks
-// the group's 32-key tiles with every f32 product as three fp16 ones
-// (hi*hi + hi*lo + lo*hi, f32 accumulation):
-//   S^T (2 x 16 keys x 16 queries) = K_tile Q^T     (48 MFMA 16x16x32)
-//   O^T (256 x 16)                += V_tile^T P^T   (48 MFMA 16x16x32)
-// About 1,800 matrix-core cycles per wave and tile instead of 8,192 in f32, with
-// the vector work beside them (f32 MFMAs exclude it). Q is normalized and
-// rotated once into registers (hi + lo, 64 of them) and O^T stays there (64).
-// The tile's planes (jeff_k_prep_split_kernel) come by LDS-DMA into one K and
-// one V buffer: K of the next tile is loaded during the softmax and P.V, V
-// during the scores, so 64 KB serve a workgroup and two of them share a CU:
-// one's loads of Q (a burst of the whole tensor over all CUs: 4-5 us), waits and
-// output stores run beside the other's products. Two buffers of each with one
-// workgroup per CU measured 45 us against 39 at 16 rows x 256 and 49 against 46
-// at 5 x 333; eight waves sharing a tile 45. Stamps of a tile (cycles): scores
-// 1,500-1,800, softmax 500-750, P.V 1,200, waits and barriers about 450.
-// Measured with the prep: 16 rows x 256 left-padded 48-54 -> 39 us, 5 rows x 333
-// 108 -> 46 us (it ran element loads without this path).
+// the group's 32-key tiles with every f32 product as six bf16 ones
+// (split_bf16x3, f32 accumulation):
+//   S^T (2 x 16 keys x 16 queries) = K_tile Q^T     (96 MFMA 16x16x32)
+//   O^T (256 x 16)                += V_tile^T P^T   (96 MFMA 16x16x32)
+// 3,072 matrix-core cycles per wave and tile instead of 8,192 in f32, with
+// the vector work beside them (f32 MFMAs exclude it); the operands of eight waves
+// take 6,144 cycles of a CU's LDS reads, as long as its matrix cores need. The
+// pieces hold all 24 bits over f32's exponent range, and a key's depend on
+// that key alone: masked, future and improbable keys of any magnitude stay out of
+// the others' way (fp16 pairs with a scale per tile need half the products, but do
+// not have that property). Q is normalized and rotated once into registers (96 of
+// them) and O^T stays there (64). The tile's planes (jeff_k_prep_split_kernel) come
+// by LDS-DMA in four pieces of 24 KB through a ring of three, two pieces ahead of
+// their use, so 75 KB serve a workgroup and two of them share a CU: one's loads of Q
+// (a burst of the whole tensor over all CUs: 4-5 us), waits and output stores run
+// beside the other's products. Cycles of a wave: Q 9,000-14,000, its norm and split
+// 4,200-5,000, the first tile's arrival 2,500, a tile 6,900 alone on its SIMD and 7,800
+// with another wave (3,260 of matrix-core time each), the gate and output 10,000-11,000.
+// Measured with the prep (f32 MFMA -> fp16 pairs -> this): 16 rows x 256 left-padded
+// 48-51 -> 39 -> 48 us, 5 rows x 333 108 -> 46 -> 57 us; relative error against 64
+// bits 2.0e-7 -> 2.0e-7 -> 1.5e-7 and 2.9e-7 -> 2.1e-7 -> 1.6e-7. A ring of six with one
+// workgroup per CU: 65 and 62 us.
 //
 // Workgroups are numbered from the last query tile down, so the longest
 // causal walks start first; the workgroups of one (row, kv head) share an id
 // residue mod 8 (one XCD, one L2) when rows x kv heads is a multiple of 8.
 template <int HDP>
 __global__ __launch_bounds__(256, 2) void jeff_split_f32_kernel(
-    const JeffArgs a, const unsigned char *__restrict__ planes, const int *__restrict__ vexp,
-    const int *__restrict__ spans, const uint32_t *__restrict__ kbits, int rows) {
-  static_assert(HDP == 256, "plane layout of 64 KB tiles");
+    const JeffArgs a, const unsigned char *__restrict__ planes, const int *__restrict__ spans,
+    const uint32_t *__restrict__ kbits, int rows) {
+  static_assert(HDP == 256, "plane layout of 96 KB tiles");
   constexpr int NB = HDP / 16, ST = HDP / 32;
   // Per wave: the redo's rows (512 + 16 * (HDP + 4) floats), of which the Q
-  // prep and the output use 16 * (HDP + 4). The K and V buffers alias them.
+  // prep and the output use 16 * (HDP + 4). The ring of pieces aliases them.
   constexpr int WROWS = 512 + 16 * (HDP + 4);
-  constexpr int PW = 8;  // 1 KB pieces of a half tile (K or V) per wave
-  static_assert(4 * WROWS * 4 >= kJeffTileBytes, "the tile buffers alias the wave rows");
+  constexpr int RING = 3, PW = kJeffPieceBytes / 4096;  // 1 KB loads of a piece per wave
+  static_assert(4 * WROWS * 4 >= RING * kJeffPieceBytes, "the ring aliases the wave rows");
   __shared__ __attribute__((aligned(16))) float smem[4 * WROWS];
   unsigned char *const lds = reinterpret_cast<unsigned char *>(smem);
   const int lane = threadIdx.x & 63;
@@ -1207,7 +1182,6 @@ __global__ __launch_bounds__(256, 2) void jeff_split_f32_kernel(
   float *OUT = a.out + row * a.q_row + (size_t)head * hd * L;
   const int nt = (L + 31) / 32;
   const unsigned char *unit = planes + (size_t)kvu * nt * kJeffTileBytes;
-  const int *uexp = vexp + (size_t)kvu * nt;
   const uint32_t *rbits = kbits + (size_t)row * nt;
 
   // The Q tile and its norm weights: issued first (wasted only for a tile
@@ -1244,9 +1218,8 @@ __global__ __launch_bounds__(256, 2) void jeff_split_f32_kernel(
   float m = kNoMax, l = 0.0f;  // l: this lane's share of the row sum
   bool tainted = false;        // wave-uniform
   if (t_begin < t_end) {
-    f16x8 qh[ST], ql[ST];
-    const int eq = spans[-2], en = eq + spans[-1];
-    const float c1 = ldexpf(a.c1, en - 2 * kJeffNormUp);
+    bf16x8 qp[3][ST];
+    const float c1 = a.c1;
     {
       // RMSNorm (lib.rs:676-691) and partial RoPE (692-709): the queries
       // transposed through the wave's LDS rows into the B operands' order,
@@ -1316,96 +1289,97 @@ __global__ __launch_bounds__(256, 2) void jeff_split_f32_kernel(
         for (int c = 0; c < 2 * ST; ++c)
           qx[c] = *reinterpret_cast<const f32x4 *>(qr + 32 * (c / 2) + 8 * grp + 4 * (c & 1));
       }
-      const float sc = pow2i(kJeffNormUp - eq);
 #pragma unroll
-      for (int c = 0; c < 2 * ST; ++c) {
-        f16x4 h, lo;
-        split_f16(qx[c], sc, h, lo);
+      for (int x = 0; x < ST; ++x) {
+        const Bf16x3 lo = split_bf16x3(qx[2 * x]), hi = split_bf16x3(qx[2 * x + 1]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          qh[c / 2][4 * (c & 1) + e] = h[e];
-          ql[c / 2][4 * (c & 1) + e] = lo[e];
-        }
+        for (int i = 0; i < 3; ++i) qp[i][x] = join_bf16(lo, hi, i);
       }
     }
-    __syncthreads();  // the wave rows become the tile buffers
+    __syncthreads();  // the wave rows become the ring
 
-    // This wave's share of a half tile's 32 pieces of 1 KB (half 0: K, 1: V).
-    auto load_half = [&](int t, int half) {
-      const u32x4r r = rsrc_words(unit + (size_t)t * kJeffTileBytes + half * kJeffTileV, kJeffTileV);
-      unsigned char *dst = lds + half * kJeffTileV;
+    // Piece p of the walk (piece p % 4 of tile t_begin + p / 4) goes to ring slot
+    // p % RING: this wave's share of its 1 KB loads.
+    const int pieces = 4 * (t_end - t_begin);
+    const unsigned char *const first_piece = unit + (size_t)t_begin * kJeffTileBytes;
+    const uint32_t voff = 16 * lane + 1024 * PW * wave;
+    int ahead = 0;                // the next piece to load
+    unsigned char *fill = lds;    // its slot
+    auto load_piece = [&] {
+      const u32x4r r = rsrc_words(first_piece + (size_t)ahead * kJeffPieceBytes, kJeffPieceBytes);
 #pragma unroll
       for (int i = 0; i < PW; ++i)
-        load_lds16(r, 16u * lane, (uint32_t)(1024 * (PW * wave + i)), dst + 1024 * (PW * wave + i));
+        load_lds16(r, voff, (uint32_t)(1024 * i), fill + 1024 * (PW * wave + i));
+      ++ahead;
+      fill = fill == lds + (RING - 1) * kJeffPieceBytes ? lds : fill + kJeffPieceBytes;
     };
-    // This wave's loads have landed (but for its youngest half tile's when
-    // `young`) and its LDS reads are done, and so for every wave.
-    auto arrive = [&](bool young) {
-      if (young)
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PW) : "memory");
-      else
+    // The next piece has landed for every wave (one more may be in flight) and every
+    // wave's reads of the piece before it are done, whose slot is refilled. Called
+    // four times per tile by every wave.
+    const unsigned char *at = lds + (RING - 1) * kJeffPieceBytes;  // the piece in use
+    auto next_piece = [&](bool last) {
+      if (last)
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PW) : "memory");
+      // Said once more where the compiler sees it: with a scalar load possibly in
+      // flight it would wait for every LDS read before the first product.
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
+      if (ahead < pieces) load_piece();
+      at = at == lds + (RING - 1) * kJeffPieceBytes ? lds : at + kJeffPieceBytes;
     };
-    load_half(t_begin, 0);
-    load_half(t_begin, 1);
-    int EV = -126;  // O's unit is 2^EV
-    constexpr float kShift = 7.0f, kLimit = 32768.0f;  // probabilities 2^7 up, below fp16's 2^15
-    const unsigned char *const kl = lds + 16 * lane, *const vl = kl + kJeffTileV;
+    load_piece();
+    load_piece();  // a tile has four
     uint32_t word_next = rbits[t_begin];  // scalar loads, one tile ahead of their use
-    int ev_next = uexp[t_begin];
     for (int t = t_begin; t < t_end; ++t) {
-      arrive(t == t_begin);  // K of t; V of t - 1 has been read by every wave
-      if (t > t_begin) load_half(t, 1);
       const uint32_t word = word_next;
-      const int ev = ev_next;
       word_next = rbits[min(t + 1, nt - 1)];
-      ev_next = uexp[min(t + 1, nt - 1)];
       const uint32_t w = q_live ? (word & range_bits(0, q - 32 * t)) : 0u;
       const bool mine = !tainted && __ballot(w != 0u) != 0;
-      f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = s0;
-      if (mine) {
-        // Three accumulators (even steps, odd steps, cross products): fewer
-        // roundings of the whole sum than one.
-        f32x4 r0 = s0, r1 = s0, u0 = s0, u1 = s0;
-        // Operands two steps ahead of their products (an LDS read takes about
-        // as long as two steps' products when all waves read), and no product
-        // right behind one into the same accumulator (it would wait for that
-        // one's eight passes).
-        f16x8 kx[3][4];
+      // A 16-key half's scores: accumulators for h*h of even and odd steps and for
+      // the smaller products, fewer roundings of the whole sum than one, and no
+      // product right behind one into the same accumulator (it would wait for that
+      // one's eight passes). Operands two steps ahead of their products (an LDS
+      // read takes about as long as two steps' products when all waves read).
+      auto scores = [&](f32x4 &s) {
+        const unsigned char *const kl = at + 16 * lane;
+        f32x4 u = s, r[3] = {s, s, s};
+        bf16x8 kx[3][3];
         auto take = [&](int x) {
-          kx[x % 3][0] = *reinterpret_cast<const f16x8 *>(kl + 2048 * x);
-          kx[x % 3][1] = *reinterpret_cast<const f16x8 *>(kl + 2048 * (ST + x));
-          kx[x % 3][2] = *reinterpret_cast<const f16x8 *>(kl + 2048 * x + 1024);
-          kx[x % 3][3] = *reinterpret_cast<const f16x8 *>(kl + 2048 * (ST + x) + 1024);
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+            kx[x % 3][i] = *reinterpret_cast<const bf16x8 *>(kl + kJeffBlock * x + 1024 * i);
         };
         take(0);
         take(1);
 #pragma unroll
         for (int x = 0; x < ST; ++x) {
           if (x + 2 < ST) take(x + 2);
-          const f16x8 k0h = kx[x % 3][0], k1h = kx[x % 3][1], k0l = kx[x % 3][2], k1l = kx[x % 3][3];
-          r0 = mfma_16x16x32_f16(k0l, ql[x], r0);
-          r1 = mfma_16x16x32_f16(k1l, ql[x], r1);
-          if (x & 1) {
-            u0 = mfma_16x16x32_f16(k0h, qh[x], u0);
-            u1 = mfma_16x16x32_f16(k1h, qh[x], u1);
-          } else {
-            s0 = mfma_16x16x32_f16(k0h, qh[x], s0);
-            s1 = mfma_16x16x32_f16(k1h, qh[x], s1);
-          }
-          r0 = mfma_16x16x32_f16(k0h, ql[x], r0);
-          r1 = mfma_16x16x32_f16(k1h, ql[x], r1);
-          r0 = mfma_16x16x32_f16(k0l, qh[x], r0);
-          r1 = mfma_16x16x32_f16(k1l, qh[x], r1);
+          const bf16x8 (&k)[3] = kx[x % 3];
+          f32x4 &a0 = r[2 * x % 3], &a1 = r[(2 * x + 1) % 3], &a2 = r[(2 * x + 2) % 3];
+          a0 = mfma_16x16x32_bf16(k[2], qp[0][x], a0);
+          a1 = mfma_16x16x32_bf16(k[1], qp[1][x], a1);
+          if (x & 1)
+            u = mfma_16x16x32_bf16(k[0], qp[0][x], u);
+          else
+            s = mfma_16x16x32_bf16(k[0], qp[0][x], s);
+          a2 = mfma_16x16x32_bf16(k[0], qp[2][x], a2);
+          a0 = mfma_16x16x32_bf16(k[1], qp[0][x], a0);
+          a1 = mfma_16x16x32_bf16(k[0], qp[1][x], a1);
           __builtin_amdgcn_sched_barrier(0);
         }
-        s0 += u0 + r0;
-        s1 += u1 + r1;
-      }
-      arrive(false);  // V of t; K of t has been read by every wave
-      if (t + 1 < t_end) load_half(t + 1, 0);
+        s += u + (r[0] + (r[1] + r[2]));
+      };
+      f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = s0;
+      next_piece(false);
+      if (mine) scores(s0);
+      next_piece(false);
+      if (mine) scores(s1);
+      next_piece(false);
+      bool ok = mine;
+      bf16x8 pp[3];
       if (mine) {
         if (__ballot(q_live && w != 0xffffffffu) != 0) {
 #pragma unroll
@@ -1422,14 +1396,13 @@ __global__ __launch_bounds__(256, 2) void jeff_split_f32_kernel(
           e1[r] = fast_exp2(__builtin_fmaf(s1[r], c1, -m));
           rs += e0[r] + e1[r];
         }
-        bool ok = true;
-        if (__ballot(q_live && !(rs <= kLimit)) != 0) {
+        if (__ballot(q_live && !(rs <= kLazyLimit)) != 0) {
           // Move the reference where the tile max exceeds it by more than the slack.
           const float mx = fmaxf(fmaxf(fmaxf(s0[0], s0[1]), fmaxf(s0[2], s0[3])),
                                  fmaxf(fmaxf(s1[0], s1[1]), fmaxf(s1[2], s1[3])));
           const float mxs = pair_max(pair16_max(mx)) * c1;
-          const bool need = mxs > m + (kRescaleSlack + kShift);
-          const float mn = need ? mxs - kShift : m;
+          const bool need = mxs > m + kRescaleSlack;
+          const float mn = need ? mxs : m;
           rs = 0.0f;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
@@ -1450,43 +1423,47 @@ __global__ __launch_bounds__(256, 2) void jeff_split_f32_kernel(
         }
         if (ok) {
           l += rs;
-          if (ev > EV) {  // a larger unit for O; a smaller tile's goes into its probabilities
-            const float f = ldexpf(1.0f, EV - ev);
+          const Bf16x3 p0 = split_bf16x3(e0), p1 = split_bf16x3(e1);
 #pragma unroll
-            for (int j = 0; j < NB; ++j) O[j] *= f;
-            EV = ev;
-          }
-          const float f = ldexpf(1.0f, ev - EV);
-          f16x4 h0, l0, h1, l1;
-          split_f16(e0, f, h0, l0);
-          split_f16(e1, f, h1, l1);
-          const f16x8 ph = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
-          const f16x8 pl = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
-          f16x8 vx[2][8];
-          auto take = [&](int g) {  // the hi and lo blocks of features 64 g ..
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-              vx[g & 1][i] = *reinterpret_cast<const f16x8 *>(vl + 2048 * (4 * g + (i & 3)) + 1024 * (i >> 2));
-          };
-          take(0);
-#pragma unroll
-          for (int g = 0; g < NB / 4; ++g) {
-            if (g + 1 < NB / 4) take(g + 1);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) O[4 * g + i] = mfma_16x16x32_f16(vx[g & 1][i], pl, O[4 * g + i]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) O[4 * g + i] = mfma_16x16x32_f16(vx[g & 1][4 + i], ph, O[4 * g + i]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) O[4 * g + i] = mfma_16x16x32_f16(vx[g & 1][i], ph, O[4 * g + i]);
-            __builtin_amdgcn_sched_barrier(0);
-          }
+          for (int i = 0; i < 3; ++i) pp[i] = join_bf16(p0, p1, i);
         }
       }
-    }
-    __syncthreads();  // the tile buffers become wave rows again
-    const float f = pow2i(EV);
+      // O^T of features 128 half ..: two 16-feature blocks per step, their
+      // operands a step ahead; the products but h*h are summed by themselves.
+      auto values = [&](auto hv) {
+        constexpr int half = decltype(hv)::value;
+        const unsigned char *const vl = at + 16 * lane;
+        bf16x8 vx[2][6];
+        auto take = [&](int g) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j) O[j] *= f;
+          for (int i = 0; i < 6; ++i)
+            vx[g & 1][i] = *reinterpret_cast<const bf16x8 *>(vl + kJeffBlock * (2 * g + i / 3) + 1024 * (i % 3));
+        };
+        take(0);
+#pragma unroll
+        for (int g = 0; g < NB / 4; ++g) {
+          if (g + 1 < NB / 4) take(g + 1);
+          const bf16x8 (&v)[6] = vx[g & 1];
+          f32x4 &o0 = O[NB / 2 * half + 2 * g], &o1 = O[NB / 2 * half + 2 * g + 1];
+          f32x4 r0 = {0.0f, 0.0f, 0.0f, 0.0f}, r1 = r0;
+#pragma unroll
+          for (int i = 2; i >= 0; --i)
+#pragma unroll
+            for (int j = 0; i + j < 3; ++j) {
+              f32x4 &x0 = i + j ? r0 : o0, &x1 = i + j ? r1 : o1;
+              x0 = mfma_16x16x32_bf16(v[i], pp[j], x0);
+              x1 = mfma_16x16x32_bf16(v[3 + i], pp[j], x1);
+            }
+          o0 += r0;
+          o1 += r1;
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+      if (ok) values(std::integral_constant<int, 0>{});
+      next_piece(t + 1 == t_end);
+      if (ok) values(std::integral_constant<int, 1>{});
+    }
+    __syncthreads();  // the ring becomes wave rows again
   }
   if (q0 >= L) return;  // no barrier follows
 
@@ -2763,12 +2740,47 @@ __global__ __launch_bounds__(256, 2) void jeff_bf16_exact_kernel(const JeffArgs 
 // ----------------------------------------------------------------- launchers
 
 // Workspace: the prepared keys (per row and kv head, keys rounded up to 16
-// for whole 16-key blocks), then one (first, last) key
-// span per row and the rows' active-key bits (32 keys per word).
+// for whole 16-key blocks) or the split kernel's planes, then one (first, last)
+// key span per row and the rows' active-key bits (32 keys per word).
 static size_t jeff_kp_main_bytes(const JeffArgs &a, int rows, int hd_pad, bool bf16) {
   const size_t Lp = ((size_t)a.L + 15) & ~(size_t)15;
   const size_t b = (size_t)rows * a.kv_heads * Lp * hd_pad * (bf16 ? 2 : 4);
   return (b + 255) & ~(size_t)255;
+}
+
+// Which f32 kernel takes a call (also sizes its workspace).
+enum class JeffF32Path { kHalf, kFused, kSplit, kGeneral };
+
+// 16-byte accesses along tokens need L % 4 == 0 and aligned bases; buffer
+// offsets need one head's (hd, L) block and one kv head's K rows within
+// 2 GiB.
+static bool jeff_f32_vec(const JeffArgs &a, int hd_pad) {
+  const uintptr_t bases = reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.v) |
+                          reinterpret_cast<uintptr_t>(a.gate) | reinterpret_cast<uintptr_t>(a.out);
+  return a.L % 4 == 0 && (bases & 15) == 0 && ((size_t)a.L + 15) * (size_t)hd_pad * 4 < ((size_t)1 << 31);
+}
+
+// Grids of at most two workgroups per CU (one row of C4 is 128) take
+// the fused kernel: one launch, no K prep, every query tile's key range
+// on eight wavefronts; of at most half the CUs (one C4 row per call) with each
+// item as two workgroups, one per half of the output features. Larger grids
+// take the prep and the split kernel, whose tiles are normalized and split once
+// instead of for every query tile. It takes every length and alignment (its
+// 16-byte accesses along tokens need dword alignment only); its buffer offsets
+// need one head's (hd, L) block within 2 GiB.
+static JeffF32Path jeff_f32_path(const JeffArgs &a, int rows, int hd_pad) {
+  const bool div_ok = (uint64_t)rows * a.heads * a.heads <= ((uint64_t)1 << 32);
+  if (hd_pad != 256 || !div_ok) return JeffF32Path::kGeneral;
+  const int rb = a.cos_t == nullptr ? 0 : (a.rot_half % 16 == 0 ? a.rot_half / 16 : -1);
+  const long items = (long)((a.L + kJeffWaveQueries - 1) / kJeffWaveQueries) * rows * a.heads;
+  const long cus = a.cus > 0 ? a.cus : 1;
+  if (jeff_f32_vec(a, hd_pad) && a.hd == 256 && rb >= 0 && rb <= 2) {
+    if (a.L <= kJeffHalfMaxL && 2 * items <= cus) return JeffF32Path::kHalf;
+    if (items <= 2 * cus) return JeffF32Path::kFused;
+  }
+  return ((size_t)a.L + 15) * (size_t)hd_pad * 4 < ((size_t)1 << 31) && a.kv_heads <= 32767
+             ? JeffF32Path::kSplit
+             : JeffF32Path::kGeneral;
 }
 
 template <int HDP>
@@ -2781,26 +2793,10 @@ static hipError_t launch_jeff_f32_hd(const JeffArgs &a, int rows, float *kp, hip
   const int pairs_per_group = kJeffF32Waves / a.heads_per_group / 2;
   const int npairs = (nq + 1) / 2;
   dim3 grid((npairs + pairs_per_group - 1) / pairs_per_group, a.heads / a.heads_per_group, rows);
-  // 16-byte accesses along tokens need L % 4 == 0 and aligned bases; buffer
-  // offsets need one head's (hd, L) block and one kv head's K rows within
-  // 2 GiB.
-  const uintptr_t bases = reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.v) |
-                          reinterpret_cast<uintptr_t>(a.gate) | reinterpret_cast<uintptr_t>(a.out);
-  const bool vec = a.L % 4 == 0 && (bases & 15) == 0 &&
-                   ((size_t)a.L + 15) * (size_t)HDP * 4 < ((size_t)1 << 31);
   if constexpr (HDP == 256) {
-    // Grids of at most two workgroups per CU (one row of C4 is 128) take
-    // the fused kernel: one launch, no K prep, every query tile's key range
-    // on eight wavefronts. Larger grids take the prep and the split
-    // kernel, whose tiles are normalized and split once instead of for
-    // every query tile.
-    const int rb = a.cos_t == nullptr ? 0 : (a.rot_half % 16 == 0 ? a.rot_half / 16 : -1);
-    const long items = (long)nq * rows * a.heads;
-    const bool div_ok = (uint64_t)rows * a.heads * a.heads <= ((uint64_t)1 << 32);
-    // Grids of at most half the CUs (one C4 row per call) run each item as
-    // two workgroups, one per half of the output features.
-    if (vec && div_ok && a.hd == 256 && rb >= 0 && rb <= 2 && a.L <= kJeffHalfMaxL &&
-        2 * items <= (a.cus > 0 ? a.cus : 1)) {
+    const JeffF32Path path = jeff_f32_path(a, rows, HDP);
+    const int rb = a.cos_t == nullptr ? 0 : a.rot_half / 16;
+    if (path == JeffF32Path::kHalf) {
       const dim3 hgrid((unsigned)(rows * a.heads), (unsigned)nq, 2u);
       void (*const kern[3][2])(JeffArgs, int) = {
           {jeff_fused_half_f32_kernel<0, false>, jeff_fused_half_f32_kernel<0, true>},
@@ -2810,8 +2806,7 @@ static hipError_t launch_jeff_f32_hd(const JeffArgs &a, int rows, float *kp, hip
                             ev.stop, 0, a, rows);
       return hipGetLastError();
     }
-    if (vec && div_ok && a.hd == 256 && rb >= 0 && rb <= 2 &&
-        items <= 2L * (a.cus > 0 ? a.cus : 1)) {
+    if (path == JeffF32Path::kFused) {
       constexpr int NW = kJeffFusedWaves;
       const dim3 fgrid((unsigned)(rows * a.heads), (unsigned)nq);
       if (rb == 0)
@@ -2825,25 +2820,20 @@ static hipError_t launch_jeff_f32_hd(const JeffArgs &a, int rows, float *kp, hip
                               ev.start, ev.stop, 0, a, rows);
       return hipGetLastError();
     }
-    // The split kernel takes every length and alignment (its 16-byte accesses
-    // along tokens need dword alignment only); buffer offsets need one head's
-    // (hd, L) block within 2 GiB.
-    if (((size_t)a.L + 15) * (size_t)HDP * 4 < ((size_t)1 << 31) && div_ok &&
-        a.kv_heads <= 32767) {
+    if (path == JeffF32Path::kSplit) {
       const int nt = (a.L + 31) / 32;
       const size_t tiles = (size_t)rows * a.kv_heads * nt;
       unsigned char *planes = reinterpret_cast<unsigned char *>(kp);
-      int *vexp = reinterpret_cast<int *>(planes + tiles * kJeffTileBytes);
-      int *spans = vexp + tiles + 2;
+      int *spans = reinterpret_cast<int *>(planes + tiles * kJeffTileBytes);
       uint32_t *kbits = reinterpret_cast<uint32_t *>(spans + 2 * rows);
       hipExtLaunchKernelGGL(jeff_k_prep_split_kernel, dim3(nt, 2 * a.kv_heads, rows), dim3(256), 0,
-                            stream, ev.start, nullptr, 0, a, planes, vexp, spans, kbits);
+                            stream, ev.start, nullptr, 0, a, planes, spans, kbits);
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
       const unsigned units = (unsigned)(rows * a.kv_heads * (a.groups / a.heads_per_group));
       const unsigned n4 = (unsigned)((nq * a.heads_per_group + 3) / 4);
       hipExtLaunchKernelGGL((jeff_split_f32_kernel<HDP>), dim3(units, n4), dim3(256), 0, stream,
-                            nullptr, ev.stop, 0, a, planes, vexp, spans, kbits, rows);
+                            nullptr, ev.stop, 0, a, planes, spans, kbits, rows);
       return hipGetLastError();
     }
   }
@@ -2852,7 +2842,7 @@ static hipError_t launch_jeff_f32_hd(const JeffArgs &a, int rows, float *kp, hip
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const dim3 block(kJeffF32Waves * 64);
-  if (vec)
+  if (jeff_f32_vec(a, HDP))
     hipExtLaunchKernelGGL((jeff_attention_f32_kernel<HDP, true>), grid, block, 0, stream, nullptr,
                           ev.stop, 0, a, kp);
   else
@@ -2884,10 +2874,10 @@ size_t jeff_kp_bytes(const JeffArgs &a, int rows, int hd_pad, bool bf16) {
   if (bf16 && hd_pad == 256 && jeff_bf16_wide_fits(a))
     return jeff_bf16_flags_offset(a, rows) + jeff_bf16_wide_flag_count(a, rows) * sizeof(int);
   const size_t nt = ((size_t)a.L + 31) / 32;
-  const size_t main = jeff_kp_main_bytes(a, rows, hd_pad, bf16);
-  const size_t tiles = (size_t)rows * a.kv_heads * nt;  // f32 at hd 256: planes and V exponents
-  const size_t split = !bf16 && hd_pad == 256 ? tiles * (kJeffTileBytes + sizeof(int)) + 2 * sizeof(int) : 0;
-  return (main > split ? main : split) + (size_t)rows * 2 * sizeof(int) +
+  const size_t keys = !bf16 && jeff_f32_path(a, rows, hd_pad) == JeffF32Path::kSplit
+                          ? (size_t)rows * a.kv_heads * nt * kJeffTileBytes
+                          : jeff_kp_main_bytes(a, rows, hd_pad, bf16);
+  return keys + (size_t)rows * 2 * sizeof(int) +
          (size_t)rows * nt * sizeof(uint32_t);
 }
 
@@ -2955,3 +2945,4 @@ hipError_t launch_jeff_attention_bf16(const JeffArgs &a, int rows, int hd_pad, v
 }
 
 }  // namespace tfd
+

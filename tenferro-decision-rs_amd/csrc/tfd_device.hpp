@@ -12,7 +12,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
 
@@ -248,25 +247,6 @@ __device__ __forceinline__ Bf16x3 split_bf16x3(f32x4 v) {
 __device__ __forceinline__ bf16x8 join_bf16(const Bf16x3 &lo, const Bf16x3 &hi, int i) {
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo.p[i], hi.p[i], 0, 1, 2, 3));
 }
-
-// v * scale (a power of two) as hi + lo fp16: hi = fp16(v), lo = fp16(v -
-// hi), 22 significant bits while |v| lies in fp16's range (lo is exact to
-// 2^-25 below it). Two mixed-precision fused operations per element.
-__device__ __forceinline__ void split_f16(f32x4 v, float scale, f16x4 &hi, f16x4 &lo) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    hi[i] = (_Float16)__builtin_fmaf(v[i], scale, 0.0f);
-    lo[i] = (_Float16)__builtin_fmaf(v[i], scale, -(float)hi[i]);
-  }
-}
-__device__ __forceinline__ void split_f16(f32x4 v, f16x4 &hi, f16x4 &lo) {
-  hi = __builtin_convertvector(v, f16x4);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) lo[i] = (_Float16)__builtin_fmaf(v[i], 1.0f, -(float)hi[i]);
-}
-
-// 2^e as f32 for e in [-126, 127].
-__device__ __forceinline__ float pow2i(int e) { return __uint_as_float((uint32_t)(127 + e) << 23); }
 
 __device__ __forceinline__ int wave_min(int v) {
 #pragma unroll
