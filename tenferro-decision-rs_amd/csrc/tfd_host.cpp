@@ -62,7 +62,7 @@ struct tfd_ctx {
   DevBuf kp;          // Jeff normalized + rotated keys
   DevBuf layer;       // intermediates of the layer entries (projections, attention output)
   DevBuf model;       // activations and token inputs of the model forward
-  DevBuf planes;      // fp16 planes of the linears' operands
+  DevBuf planes;      // bf16 planes of the linears' operands
   std::vector<uint8_t> model_host;  // packed token inputs of the last model forward
   bool model_inflight = false;      // an asynchronous forward may still read model_host
   rocblas_handle blas = nullptr;  // the layer entries' GEMMs, on `stream`
@@ -653,12 +653,12 @@ int gemm(tfd_ctx *c, bool ta, bool tb, size_t m, size_t n, size_t k, const float
   return TFD_OK;
 }
 
-// ------------------------------------------- linears on fp16 planes
+// ------------------------------------------- linears on bf16 planes
 
 // An operand's planes (split_gemm.hip): `rows` rows of k elements.
 struct Planes {
   unsigned char *p = nullptr;
-  int *exps = nullptr;
+  int *marks = nullptr;
   size_t rows = 0, k = 0;
   size_t half = 0;  // > 0: GeGLU weights of 2 * half rows, 16-row blocks alternating
   size_t blocks() const {
@@ -677,7 +677,7 @@ int reserve_planes(tfd_ctx *c, std::initializer_list<Planes *> list) {
   unsigned char *at = static_cast<unsigned char *>(c->planes.ptr);
   for (Planes *p : list) {
     p->p = at;
-    p->exps = reinterpret_cast<int *>(at + ((p->bytes() + 255) & ~(size_t)255));
+    p->marks = reinterpret_cast<int *>(at + ((p->bytes() + 255) & ~(size_t)255));
     at += p->total();
   }
   return TFD_OK;
@@ -693,7 +693,7 @@ tfd::SplitSeg split_seg(const Planes &d, const float *src, const int *map = null
   g.src = src;
   g.map = map;
   g.dst = d.p;
-  g.exps = d.exps;
+  g.marks = d.marks;
   g.rows = (int)d.rows;
   g.k = (int)d.k;
   g.blocks = (int)d.blocks();
@@ -711,24 +711,31 @@ int split_rows(tfd_ctx *c, std::initializer_list<tfd::SplitSeg> list) {
   return TFD_OK;
 }
 
-// Whether a linear of `cols` columns (weights out x in) runs as fp16 planes:
-// from the size where splitting both operands on each call (5 us or more) plus the
-// three fp16 products undercut one f32 product, and a size the planes'
-// 32-bit indices hold. Whole layers, f32 products -> planes: Laya hidden 512 at
-// 1024 columns 61 -> 67 us and at 1400 102 -> 87; 768 at 896 84 -> 79; 1024 at
-// 512 63 -> 74 and at 640 87 -> 82; Jeff hidden 1024 at 512 91 -> 108 and at
-// 640 139 -> 113.
-bool split_pays(size_t out, size_t in, size_t cols) {
-  return in >= 256 && out >= 256 && cols >= 640 && out * cols >= ((size_t)5 << 17) &&
-         in <= 65536 && out <= ((size_t)1 << 26) && cols <= ((size_t)1 << 26);
+// Whether a linear of `cols` columns (weights out x in) runs as bf16 planes:
+// from the size where splitting both operands on each call (5 us or more each, by
+// the weights' and the columns' size) plus the six bf16 products undercut one f32
+// product, and a size the planes' 32-bit indices hold. Whole layers, f32 products ->
+// planes: Laya hidden 256 at 8192 columns 59 -> 72 us, 384 at 3072 56 -> 65, 512 at
+// 2048 55 -> 61 and at 3072 77 -> 77; 768 at 1280 65 -> 77, at 1536 88 -> 89 and at
+// 2048 108 -> 95; 1024 at 1024 80 -> 90 and at 1536 122 -> 112; 2048 at 256 104 -> 128
+// and at 384 162 -> 154; Jeff hidden 1024 (2048 features) at 512 82 -> 114, at 640
+// 137 -> 130, at 1024 142 -> 147 and at 2048 280 -> 214.
+constexpr double kLayerSplit = 9.0 * (1 << 27);
+// The forward's norms write planes by themselves: 4 layers of hidden 768 at 1024
+// columns 919 -> 921 us, at 1280 973 -> 974 and at 1536 1167 -> 1063; 1024 at 640 1213 ->
+// 1257 and at 896 1589 -> 1386; 512 at 1536 725 -> 738 and at 2048 815 -> 798.
+constexpr double kForwardSplit = 6.0 * (1 << 27);
+bool split_pays(size_t out, size_t in, size_t cols, double products) {
+  return in >= 512 && out >= 512 && cols >= 384 && in <= 65536 && out <= ((size_t)1 << 26) &&
+         cols <= ((size_t)1 << 26) && (double)in * (double)out * (double)cols >= products;
 }
 
 tfd::SplitGemmArgs split_args(const Planes &a, const Planes &b, size_t m) {
   tfd::SplitGemmArgs g{};
   g.a = a.p;
   g.b = b.p;
-  g.ea = a.exps;
-  g.eb = b.exps;
+  g.ma = a.marks;
+  g.mb = b.marks;
   g.m = (int)m;
   g.n = (int)b.rows;
   g.nkb = (int)((a.k + 31) / 32);
@@ -769,7 +776,7 @@ int laya_layer_dev(tfd_ctx *c, const char *op, const float *x, size_t hidden, si
   // Workspace: qkv (3d, L, B), then the attention output (d, L, B).
   if ((rc = reserve(c, c->layer, sizeof(float) * 4 * n))) return rc;
   float *qkv = static_cast<float *>(c->layer.ptr), *att = qkv + 3 * n;
-  if (split_pays(hidden, hidden, tokens)) {
+  if (split_pays(hidden, hidden, tokens, kLayerSplit)) {
     Planes wi, wo, xp;
     wi.rows = 3 * hidden;
     wo.rows = hidden;
@@ -889,7 +896,7 @@ int jeff_layer(tfd_ctx *c, size_t rows, size_t length, size_t hidden, size_t hea
                     (flags & TFD_TRIM_LEADING) | TFD_DEVICE_PTRS | TFD_ASYNC);
   };
   const size_t tokens = rows * length;
-  if (split_pays(W, hidden, tokens) && split_pays(hidden, W, tokens)) {
+  if (split_pays(W, hidden, tokens, kLayerSplit) && split_pays(hidden, W, tokens, kLayerSplit)) {
     // One product for the four projections: their weights' planes follow one
     // another (each padded to whole 16-row blocks), tokens are the rows.
     auto pad = [](size_t n) { return 16 * tfd::split_blocks(n); };
@@ -911,7 +918,7 @@ int jeff_layer(tfd_ctx *c, size_t rows, size_t length, size_t hidden, size_t hea
       Planes part = wp;
       part.rows = n4[i];
       part.p = wp.p + at / 16 * ((hidden + 31) / 32) * tfd::kSplitBlock;
-      part.exps = wp.exps + at;
+      part.marks = wp.marks + at;
       s4[i] = split_seg(part, w4[i]);
       ga.outs[i] = tfd::SplitOut{y4[i], (int)at, (int)n4[i]};
       at += pad(n4[i]);
@@ -1190,9 +1197,10 @@ int laya_forward(tfd_ctx *c, const tfd_laya_model *m, const int64_t *ids, const 
         *a1 = take(AH * B);
   const bool dev_out = (flags & TFD_DEVICE_PTRS) != 0;
   float *act_d = dev_out ? action : take(A * B), *log_d = dev_out ? logits : take(KB);
-  // Long batches: the layers' linears on fp16 planes, split layer by layer.
+  // Long batches: the layers' linears on bf16 planes, split layer by layer.
   // Columns that are normalized first are written as planes by the norm.
-  const bool split = split_pays(d, d, Tc) && (m->n_layers == 0 || split_pays(d, I, Tc)) &&
+  const bool split = split_pays(d, d, Tc, kForwardSplit) &&
+                     (m->n_layers == 0 || split_pays(d, I, Tc, kForwardSplit)) &&
                      tfd::norm_split_fits((int)d);
   Planes p_qkv, p_wo, p_wi, p_wm, p_x, p_g;  // weights, d-wide columns, wider columns
   if (split) {
@@ -1259,7 +1267,7 @@ int laya_forward(tfd_ctx *c, const tfd_laya_model *m, const int64_t *ids, const 
     na.ldx = na.d = (int)d;
     na.per = 1;
     na.eps = eps;
-    TFD_HIP(c, tfd::launch_norm_split(na, p_x.p, p_x.exps, c->stream), "norm launch");
+    TFD_HIP(c, tfd::launch_norm_split(na, p_x.p, p_x.marks, c->stream), "norm launch");
     return (int)TFD_OK;
   };
   // The attention block on p_x's columns with p_qkv and p_wo, added into res.

@@ -248,10 +248,10 @@ hipError_t launch_pool(const PoolArgs &a, int batch, hipStream_t stream);
 hipError_t launch_copy_columns(const float *src, const int *src_map, float *dst,
                                const int *dst_map, int m, long n, hipStream_t stream);
 
-// ------------------------------------------------ f32 linears on fp16 planes
+// ------------------------------------------------ f32 linears on bf16 planes
 
-// Bytes of one plane block: 16 rows x 32 k, hi then lo (split_gemm.hip).
-constexpr int kSplitBlock = 2048;
+// Bytes of one plane block: 16 rows x 32 k, three pieces (split_gemm.hip).
+constexpr int kSplitBlock = 3072;
 inline size_t split_blocks(size_t rows) { return (rows + 15) / 16; }
 inline size_t split_plane_bytes(size_t rows, size_t k) {
   return split_blocks(rows) * ((k + 31) / 32) * kSplitBlock;
@@ -262,7 +262,7 @@ struct SplitSeg {
   const float *src;
   const int *map;      // or null: plane row p reads source row map[p]
   unsigned char *dst;  // split_plane_bytes
-  int *exps;           // 16 * blocks
+  int *marks;          // 16 * blocks: rows that hold an inf or NaN
   int rows, k, blocks;
   int length;          // trans: tokens per question row
   int half;            // > 0: alternate 16-row blocks of rows 0.. and half.. (GeGLU)
@@ -287,7 +287,7 @@ struct SplitOut {
 };
 struct SplitGemmArgs {
   const unsigned char *a, *b;  // planes
-  const int *ea, *eb;
+  const int *ma, *mb;          // marks
   int m, n, nkb;     // outputs along A (kEpiGeglu: one half's), columns, 32-k blocks
   int mrows;         // plane rows of A (kEpiGeglu: both halves, padded to 16)
   int mt, nt;        // tiles (set by the launcher)
@@ -303,7 +303,7 @@ struct SplitGemmArgs {
 hipError_t launch_split_gemm(const SplitGemmArgs &g, int epi, int cus, hipStream_t stream);
 // LayerNorm (a.y, a.add unused) straight into planes; d as norm_split_fits says.
 bool norm_split_fits(int d);
-hipError_t launch_norm_split(const NormArgs &a, unsigned char *dst, int *exps,
+hipError_t launch_norm_split(const NormArgs &a, unsigned char *dst, int *marks,
                              hipStream_t stream);
 
 // ------------------------------------------------ f32 linears over few columns

@@ -1,8 +1,8 @@
 """Checks on the gfx950 assembly of the kernels that use LDS-DMA loads (CPU
 only: hipcc cross-compiles without a GPU).
 
-The bf16 wide kernel's K/V tiles and the f32 split-head kernel's prefetched
-K/V slices and gate arrive through inline-assembly LDS-DMA loads
+The bf16 wide kernel's K/V tiles, the f32 split kernel's K/V pieces and the
+plane products' operands arrive through inline-assembly LDS-DMA loads
 (`buffer_load_dwordx4 ... lds`) whose LDS address comes from M0. The asm
 writes M0 itself without naming it as clobbered, because the compiler
 reserves M0 and ignores such a clobber. That is only sound while the
@@ -26,8 +26,8 @@ HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 KERNELS = [
     ("jeff_bf16_wide.hip", "_ZN3tfd21jeff_bf16_wide_kernel"),
     ("jeff_attention.hip", "_ZN3tfd21jeff_split_f32_kernelILi256E"),
-    ("split_gemm.hip", "_ZN3tfd12_GLOBAL__N_117split_gemm_kernelILi128ELi128E"),
-]
+] + [("split_gemm.hip", f"_ZN3tfd12_GLOBAL__N_117split_gemm_kernelILi64ELi{bn}ELi{epi}E")
+     for bn in (64, 128) for epi in range(3)]  # every tile and epilogue
 
 
 @pytest.fixture(scope="module")
@@ -66,7 +66,7 @@ def _body(lines, prefix):
     return out
 
 
-@pytest.mark.parametrize("src,prefix", KERNELS, ids=[k[0] for k in KERNELS])
+@pytest.mark.parametrize("src,prefix", KERNELS, ids=[k[1] for k in KERNELS])
 def test_m0_only_feeds_the_lds_dma_loads(asm_of, src, prefix):
     code = _body(asm_of(src), prefix)
     m0 = re.compile(r"\bm0\b")
