@@ -1,12 +1,11 @@
 """Laya attention with keys and values whose magnitude changes from tile to
-tile (the fp16 split of the aligned path keeps one power-of-two scale per tile
-and takes it anew only when a tile leaves its range): jumps up and down by far
-more than fp16 holds, all-zero tiles, a tile with an inf that is never kept,
-in both entries, for every workgroup shape (teams of two and four waves, one
-team) and head dim of that path. The expectation is the oracle, which takes its
-RoPE angles in f32 as the op does (64-bit brute force does not: at position
-417 an angle differs by up to 417 * 2^-24, and scores of order 30 by as much
-times that, far above the tolerance). An output is a convex combination of kept
+tile: jumps up and down by far more than a half-precision number holds, all-zero
+tiles, a tile with an inf that is never kept, in both entries, for every
+workgroup shape (teams of two and four waves, one team) and head dim of the
+aligned path (test_laya_ranges has the jumps inside a tile). The expectation is
+the oracle, which takes its RoPE angles in f32 as the op does (64-bit brute force
+does not: at position 417 an angle differs by up to 417 * 2^-24, and scores of
+order 30 by as much times that, far above the tolerance). An output is a convex combination of kept
 values, so the tolerance is 2e-5 of the largest value a query keeps (its
 window), the f32 tolerance at that scale.
 """
