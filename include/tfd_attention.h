@@ -229,8 +229,8 @@ int tfd_jeff_full_attention_rows_bf16(tfd_ctx *ctx, size_t rows, size_t length, 
  *   w_in:   (hidden, 3*hidden) column-major, element i + hidden*o; b_in (3*hidden) or NULL.
  *   w_out:  (hidden, hidden) column-major; b_out (hidden) or NULL.
  *   keep:   (L, L, B) bytes as for tfd_laya_attention_block_f32.
- * The linears are f32 (large ones as three fp16 products per f32 product,
- * small ones as f32 GEMMs) on the context's stream; the
+ * The linears are f32 (large ones as six bf16 products per f32 product, which
+ * keep every operand's 24 bits, small ones as f32 GEMMs) on the context's stream; the
  * intermediates live in the context's workspace.
  */
 int tfd_laya_attention_layer_f32(tfd_ctx *ctx, const float *x, size_t hidden, size_t heads,

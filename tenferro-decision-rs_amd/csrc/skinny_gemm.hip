@@ -9,7 +9,8 @@
 // matrix cores' layout), and the eight partial sums meet once in LDS. LayerNorm
 // of the columns (their elements are in the waves' registers anyway), the
 // gather of the columns, bias, activation, GeGLU, residual add and the scatter
-// of the result are part of it. Measured at 96 columns (768 -> 2304): 14.8 us
+// of the result are part of it. Linears of more than 768 inputs come here up to 64
+// columns only (f32 GEMMs beyond). Measured at 96 columns (768 -> 2304): 14.8 us
 // with LayerNorm and scatter, against 16 us for the f32 GEMM plus 7 us for the
 // LayerNorm and 4 us for the column move; 768 -> 768 12.7 us against 11 + 4. What
 // remains is the chain of dependent round trips: arguments, column map,

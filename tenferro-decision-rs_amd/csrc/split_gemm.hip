@@ -54,8 +54,9 @@ __device__ __forceinline__ void write_split8(unsigned char *p, const float (&x)[
 }
 
 // One workgroup = 16 rows of one operand; its 8 waves take the 32-k blocks in
-// turn, U of them in flight. Bound by HBM: 4 bytes read and 6 written per
-// element. Source rows: contiguous in k (one lane reads 32 bytes of a row, a wave
+// turn, U of them in flight (4: 32 us for 4096 x 1024 token-contiguous with 7.3 M weights,
+// 26 for 4096 x 2048; 8: 34 and 28, 2: 38 and 24). Bound by HBM: 4 bytes read and 6
+// written per element. Source rows: contiguous in k (one lane reads 32 bytes of a row, a wave
 // whole 128-byte lines), or transposed (SplitSeg::trans: 16 consecutive tokens per
 // k). Anything unaligned or ragged goes element by element.
 template <int U>
@@ -246,9 +247,10 @@ constexpr int kGroup = 8;  // A tiles per group of the tile order
 // bf16 library product reaches 1,197), ones of few tiles per CU by the loads' latency
 // (64 x 64 alone on a CU 0.45 us per step, 0.33 us each with three). Measured
 // against f32 matrix products, alone, without the splits: 2304 x 4096 x 768 112-136 ->
-// 90 us, 768 x 2309 x 1152 40 -> 26, 5120 x 4096 x 1024 353 -> 220. As fp16 pairs (half
-// the products) the first took 52 us, but their rows lose the bits of elements far
-// below the largest.
+// 90 us back to back (72 within a layer, whose other kernels leave the clocks higher),
+// 768 x 2309 x 1152 40 -> 26, 5120 x 4096 x 1024 353 -> 220 (197 within a layer). As fp16
+// pairs (half the products) the first took 52 us, but their rows lose the bits of
+// elements far below the largest.
 template <int BM, int BN, int EPI>
 __global__ __launch_bounds__(256, 2) void split_gemm_kernel(SplitGemmArgs g) {
   constexpr int TM = BM / 32, TN = BN / 32;          // 16 x 16 blocks per wave

@@ -965,8 +965,12 @@ int jeff_layer(tfd_ctx *c, size_t rows, size_t length, size_t hidden, size_t hea
 // (LayerNorm over twice the registers) at 96 2579 -> 2605, 128 2580 -> 2630.
 size_t skinny_columns(size_t in) { return in <= 768 ? 160 : 64; }
 
-// Whether a linear by itself takes the few-column kernel: the same limit (a
-// 1024-wide forward at 96 columns with its linears here one by one: 2594 -> 2998).
+// Whether a linear by itself takes the few-column kernel: the same limit by its own
+// inputs, so one of more than 768 inputs (a model's second MLP linear) is an f32 GEMM
+// above 64 columns. Forwards of 22 layers with those linears as GEMMs -> here: hidden 768
+// with 1152 inputs at 72 columns 1451 -> 1471 us, 96 1488 -> 1524, 160 2056 -> 2096, with
+// 3072 at 96 2155 -> 2285; hidden 384 with 1536 at 96 1495 -> 1449. A 1024-wide forward at
+// 96 columns with all its linears here one by one: 2594 -> 2998.
 bool skinny_fits(size_t in, size_t out, size_t cols, const float *w, const float *x) {
   return cols <= skinny_columns(in) && in % 4 == 0 && in > 0 && in <= (size_t)INT32_MAX / 4 &&
          out <= (size_t)INT32_MAX / 4 && aligned16(w) && aligned16(x);

@@ -253,15 +253,12 @@ hipError_t launch_copy_columns(const float *src, const int *src_map, float *dst,
 // Bytes of one plane block: 16 rows x 32 k, three pieces (split_gemm.hip).
 constexpr int kSplitBlock = 3072;
 inline size_t split_blocks(size_t rows) { return (rows + 15) / 16; }
-inline size_t split_plane_bytes(size_t rows, size_t k) {
-  return split_blocks(rows) * ((k + 31) / 32) * kSplitBlock;
-}
 
 // One operand to split: `blocks` plane row blocks of k elements each.
 struct SplitSeg {
   const float *src;
   const int *map;      // or null: plane row p reads source row map[p]
-  unsigned char *dst;  // split_plane_bytes
+  unsigned char *dst;  // blocks * ceil(k / 32) plane blocks
   int *marks;          // 16 * blocks: rows that hold an inf or NaN
   int rows, k, blocks;
   int length;          // trans: tokens per question row

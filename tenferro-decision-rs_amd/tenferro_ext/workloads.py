@@ -231,8 +231,8 @@ def jeff_config(cfg: int, *, rows: Optional[int] = None, length: Optional[int] =
 # ------------------------------------------------------------------ layers
 #
 # Whole-layer inputs for the layer entries: unit activations x and
-# N(0, 0.02^2) projection weights (the reading under which configs[1] and
-# configs[3] give the projections' scale used above), seeded 100 + cfg.
+# N(0, 0.02^2) projection weights (the reading under which C2 and C4
+# give the projections' scale used above), seeded 100 + cfg.
 
 
 @dataclass
