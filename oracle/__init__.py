@@ -1,7 +1,7 @@
 """TEST INFRASTRUCTURE ONLY -- CPU oracle for the fused attention path.
 
 Only tests/, ``__graft_entry__.smoke()`` and bench.py's ``cpu_baseline`` leg may
-import this package, and only as the checker or the timed CPU baseline; the
+import this package, and only as the oracle or the timed CPU baseline; the
 product (``tenferro_ext`` / ``libtfd_attention.so``) never calls into it.
 
 Two independent restatements live here:

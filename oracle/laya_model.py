@@ -1,5 +1,5 @@
 """TEST INFRASTRUCTURE ONLY -- CPU restatements of the Laya decision-model
-forward, the checker of ``tfd_laya_forward_f32``.
+forward, the oracle of ``tfd_laya_forward_f32``.
 
 * ``forward(...)``: float32 numpy, step by step as ``forward_reference``
   (crates/laya-infer/src/model.rs:867-977) and its host helpers

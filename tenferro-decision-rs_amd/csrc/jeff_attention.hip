@@ -907,7 +907,7 @@ __global__ __launch_bounds__(kJeffF32Waves * 64, 1) void jeff_attention_f32_kern
         s0[r] = fast_exp2(__builtin_fmaf(s0[r], c1, -mn));
         rs += s0[r];
       }
-      if (__ballot(q_live && !__builtin_isfinite(rs)) != 0) {
+      if (__ballot(q_live && !(__builtin_isfinite(rs) && reference_usable(mn))) != 0) {
         tainted = true;
       } else {
         if (__ballot(need) != 0) {
@@ -1410,7 +1410,7 @@ __global__ __launch_bounds__(256, 2) void jeff_split_f32_kernel(
             e1[r] = fast_exp2(__builtin_fmaf(s1[r], c1, -mn));
             rs += e0[r] + e1[r];
           }
-          if (__ballot(q_live && !__builtin_isfinite(rs)) != 0) {
+          if (__ballot(q_live && !(__builtin_isfinite(rs) && reference_usable(mn))) != 0) {
             tainted = true;
             ok = false;
           } else {
@@ -1825,7 +1825,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void jeff_fused_f32_kernel(const J
         ex[r] = fast_exp2(s[r] - mn);
         rs += ex[r];
       }
-      if (__ballot(q_live && !__builtin_isfinite(rs)) != 0) {
+      if (__ballot(q_live && !(__builtin_isfinite(rs) && reference_usable(mn))) != 0) {
         tainted = true;
       } else {
         const float alpha = fast_exp2(m - mn);  // exactly 1 where the reference stays
@@ -2248,7 +2248,7 @@ __global__ __launch_bounds__(512, 1) void jeff_fused_half_f32_kernel(const JeffA
         ex[r] = fast_exp2(s[r] - mn);
         rs += ex[r];
       }
-      if (__ballot(q_live && !__builtin_isfinite(rs)) != 0) {
+      if (__ballot(q_live && !(__builtin_isfinite(rs) && reference_usable(mn))) != 0) {
         tainted = true;
       } else {
         const float alpha = fast_exp2(m - mn);  // exactly 1 where the reference stays

@@ -417,7 +417,7 @@ __global__ __launch_bounds__(512, 1) void jeff_bf16_wide_kernel(const JeffArgs a
 #pragma unroll
       for (int i = 0; i < 8; ++i) g[i] = pack_bf16x2(e[2 * i], e[2 * i + 1]);
       rs = sum_bf16x16(g);
-      if (__ballot(q_live && !__builtin_isfinite(rs)) != 0) {
+      if (__ballot(q_live && !(__builtin_isfinite(rs) && reference_usable(mn))) != 0) {
         tainted = true;
         kw = 0;
       } else if (__ballot(mn != m) != 0) {

@@ -1021,7 +1021,7 @@ __global__ __launch_bounds__(64 * QW * TEAMS, TEAMS == 1 ? laya_groups_per_cu(HD
           e1[r] = fast_exp2(__builtin_fmaf(s1[r], c1, -mn));
           rs += e0[r] + e1[r];
         }
-        if (__ballot(qin && !__builtin_isfinite(rs)) != 0) {
+        if (__ballot(qin && !(__builtin_isfinite(rs) && reference_usable(mn))) != 0) {
           tainted = true;
           ok = false;
         } else {

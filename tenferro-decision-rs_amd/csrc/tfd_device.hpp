@@ -110,6 +110,14 @@ __device__ __forceinline__ float pair16_sum(float x) {
 constexpr float kRescaleSlack = 8.0f;
 // Initial reference: finite, so exp2(fma(-inf, c1, -m)) is exp2(-inf) = 0.
 constexpr float kNoMax = -3.402823466e38f;
+// Whether exponents can be taken as exp2(fma(s, c1, -m)) against this reference: it
+// is the rounded product of a score and c1, off by up to 2^-25 of itself, a factor that all
+// of a row's probabilities share (up to 2^8 at 2^28) until it leaves f32's range. Rows with
+// larger scores take the careful path, whose exponents are differences of rounded
+// products.
+__device__ __forceinline__ bool reference_usable(float m) {
+  return fabsf(m) <= 0x1p28f || m == kNoMax;  // kNoMax: nothing kept yet
+}
 // A lane whose 8 terms of a tile, taken against the current reference, sum
 // to at most this (2^11 = 8 * 2^kRescaleSlack) needs no new reference.
 constexpr float kLazyLimit = 2048.0f;

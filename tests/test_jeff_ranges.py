@@ -2,8 +2,9 @@
 by far more than a half-precision number's range: a masked key inside the sequence,
 left padding, a key in the causal future, a key of almost no probability before all
 others, one feature of V, and one feature of K that every query's zero meets, each
-1e6, 1e12 or 3e38 times the rest. Grids above two workgroups per CU with 4, 2 and 1
-query heads per workgroup, and one small grid.
+1e6, 1e12 or 3e38 times the rest; and norm weights that make scores past 2^24. Grids
+above two workgroups per CU with 4, 2 and 1 query heads per workgroup, one of each
+kernel for smaller grids, and a small head dim.
 
 The expectation is the same formula in 64 bits (RoPE factors from the oracle's f32
 table). An f32 evaluation is off by a few 2^-24 of sum_k p_k |v_k| of the
@@ -19,7 +20,8 @@ from tenferro_ext.workloads import Lcg
 
 THETA, EPS = 1.0e7, 1.0e-6
 SHAPES = [(5, 333, 8, 2, 256, 64), (9, 250, 4, 2, 256, 64), (6, 481, 3, 3, 256, 32),
-          (7, 289, 6, 2, 200, 50), (1, 200, 8, 2, 256, 64)]
+          (7, 289, 6, 2, 200, 50), (1, 200, 8, 2, 256, 64), (2, 200, 8, 2, 256, 64),
+          (3, 120, 4, 2, 64, 32)]
 
 
 def reference(q, k, v, gate, qn, kn, mask, rot, trim):
@@ -65,7 +67,7 @@ def inputs(R, L, H, KV, hd, case, big):
     qn, kn = normal(hd) * np.float32(0.1), normal(hd) * np.float32(0.1)
     mask = np.ones((R, L), np.float32)
     for r in range(R):
-        mask[r, :(37 * r) % (L // 2)] = 0.0
+        mask[r, :(37 * r) % max(L // 2, 1)] = 0.0
     large = np.float32(big) * (normal(2, R, KV, hd) % np.float32(1.0))
     if case == "masked":
         at = 3 * L // 4
@@ -84,6 +86,8 @@ def inputs(R, L, H, KV, hd, case, big):
             at = (37 * r) % (L // 2)
             k[r, :, hd // 2, at] = -1e4
             v[r, :, :, at] = large[1, r] * np.float32(2.0 ** -20)
+    elif case == "scores":      # far past 2^24: every query keeps its largest alone
+        qn[:], kn[:] = big, big
     elif case == "feature_v":
         v[:, :, 3] *= np.float32(big)
     else:                       # feature_k, outside the rotated ones
@@ -93,10 +97,11 @@ def inputs(R, L, H, KV, hd, case, big):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("case", ["masked", "padding", "future", "improbable", "feature_v", "feature_k"])
+@pytest.mark.parametrize("case", ["masked", "padding", "future", "improbable", "scores", "feature_v", "feature_k"])
 @pytest.mark.parametrize("rows,L,heads,kv,hd,rot", SHAPES)
 def test_ranges_gpu(gpu_ctx, rows, L, heads, kv, hd, rot, case):
-    for big in (1e6, 1e12, 3e38) if case in ("masked", "padding") else (1e6, 1e12):
+    for big in {"masked": (1e6, 1e12, 3e38), "padding": (1e6, 1e12, 3e38), "scores": (3e3, 1e5, 1e9)}.get(
+            case, (1e6, 1e12)):
         for trim in (False, True) if case == "padding" else (False,):
             print(f"[ranges] Jeff {rows} x {L}, heads {heads}/{kv} x {hd} {case} {big:g} {trim}", flush=True)
             x = inputs(rows, L, heads, kv, hd, case, big)
@@ -108,3 +113,20 @@ def test_ranges_gpu(gpu_ctx, rows, L, heads, kv, hd, rot, case):
             assert np.isfinite(err).all()
             ratio = float((err / np.maximum(size, 1e-300)).max())
             assert (err <= 2e-5 * size).all(), ratio
+
+
+@pytest.mark.gpu
+def test_bf16_scores_gpu(gpu_ctx):
+    """Rows that keep their last key alone, under norm weights of 1e5: that key's value
+    times the gate for the last query, 0 for the others."""
+    print("[ranges] Jeff bf16 scores", flush=True)
+    rows, L, heads, kv, hd = 16, 8, 8, 2, 256
+    q, k, v, gate, qn, kn, mask = inputs(rows, L, heads, kv, hd, "scores", 1e5)
+    mask[:, :L - 1], mask[:, L - 1] = 0.0, 1.0
+    bits = [te.to_bf16_bits(t.reshape(-1)) for t in (q, k, v, gate)]
+    v, gate = (te.bf16_bits_to_f32(b).astype(np.float64) for b in bits[2:])
+    want = np.repeat(v.reshape(rows, kv, hd, L), heads // kv, axis=1) / (1.0 + np.exp(-gate.reshape(rows, heads, hd, L)))
+    want[..., :L - 1] = 0.0
+    got = np.asarray(te.jeff_full_attention_rows(*bits, qn, kn, mask.reshape(-1), rows, L, heads, kv, hd, 64,
+                                                 THETA, EPS, bf16=True, ctx=gpu_ctx)).reshape(want.shape)
+    assert np.isfinite(got).all() and float(np.abs(got - want).max()) <= 1e-2

@@ -2,7 +2,7 @@
 number's range inside one 32-key tile: a masked key, a key that one query of a
 workgroup keeps, a key outside the other queries' window, one feature of V, one
 feature of K that every query's zero meets, and a key of almost no probability,
-each 1e6, 1e12 or 3e38 times the rest. For every workgroup shape (two and four
+each 1e6, 1e12 or 3e38 times the rest; and scores of that size. For every workgroup shape (two and four
 waves per team, one team) and head dim of the aligned path, both entries.
 
 The expectation is the same formula in 64 bits (RoPE factors from the oracle's f32
@@ -66,6 +66,12 @@ def inputs(hd, heads, L, B, case, big):
         keep[:, 70, :] = 0
         keep[:, 70, 75] = 1
         x[:, 70, 2] = large[1]
+    elif case == "scores":    # far past 2^24, one or two keys each
+        keep = np.zeros((B, L, L), np.uint8)
+        t = np.arange(L)
+        keep[:, t, t] = 1
+        keep[:, (t + 7) % L, t] = t % 3 > 0
+        x[:, :, :2] *= np.float32(big) ** np.float32(0.5)
     elif case == "feature_v":
         x[:, :, 2, :, 3] *= np.float32(big)
     elif case == "feature_k":  # a RoPE pair
@@ -81,11 +87,12 @@ def inputs(hd, heads, L, B, case, big):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("case", ["masked", "window", "one_query", "feature_v", "feature_k", "improbable"])
+@pytest.mark.parametrize("case", ["masked", "window", "one_query", "scores", "feature_v", "feature_k", "improbable"])
 @pytest.mark.parametrize("hd,heads,L,B", SHAPES)
 def test_ranges_gpu(gpu_ctx, hd, heads, L, B, case):
     d = hd * heads
-    for big in (1e6, 1e12, 3e38) if case in ("masked", "window") else (1e6, 1e12):
+    for big in {"masked": (1e6, 1e12, 3e38), "window": (1e6, 1e12, 3e38), "scores": (1e9, 1e12, 1e18)}.get(
+            case, (1e6, 1e12)):
         print(f"[ranges] Laya hd {hd} heads {heads} L {L} B {B} {case} {big:g}", flush=True)
         qkv, valid, window, keep = inputs(hd, heads, L, B, case, big)
         flat = np.ascontiguousarray(qkv.reshape(-1))
